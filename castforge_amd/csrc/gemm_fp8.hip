@@ -503,6 +503,225 @@ void fp8_gemm_kernel(const uint8_t *__restrict__ A, const float *__restrict__ sa
     });
 }
 
+// ---- small and mid-sized problems: K split over the waves of a workgroup ----
+//
+// `fp8_split_kernel<kExact, I, J, NW, S>`: workgroup tile 32 I (n) x 32 J (m); every wave computes
+// the whole tile over its own K chunks (chunk = 128 bytes of K, wave w takes chunks w, w + NW, ..),
+// and the NW partial tiles are summed through LDS in wave order.  The 256 x 256 kernel above is a
+// serial chain of K / 64 barriered steps on few workgroups when M or N is small.  Here a wave owns
+// its LDS ring (S stages of 32 (I + J) rows x 128 bytes), so the loop has no barrier, each wave
+// walks K / (128 NW) chunks, and up to NW S chunks per workgroup are in flight.  What bounds it: the
+// load latency of the few chunks each wave walks (small M), the L1 rate of W and A into LDS (64 x 64
+// tiles).  Measured, us, 256 x 256 kernel / this one: 4096 x 4096 at M = 24 41.1 / 8.7, M = 256
+// 45.5 / 14.9, M = 1024 48.7 / 42.1; 4096 x 11008 at M = 64 90 / 16.8; M = 512 113 / 48.6.
+// (1, 1) with 8 waves or 4 stages, (2, 1) and (1, 2) tiles were within 5 % of these two or slower.
+// Waits until at most N vector-memory loads are outstanding and every LDS read has returned, and
+// keeps memory accesses on their side of the wait (the compiler does not order LDS reads against
+// the builtin: it has moved reads of a stage above the wait for the loads that fill it).
+template <int N>
+__device__ __forceinline__ void wait_vm_fence() {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(N) & ~(15 << 8));
+    asm volatile("" ::: "memory");
+}
+
+template <bool kExact, int I, int J>
+struct SplitFrags {
+    int32x8 w[2][I], a[2][J];
+};
+
+constexpr int kSplitBK = 128;
+
+// 16-byte chunk c of row r of a 128-byte-row stage sits at c ^ ((r >> 1) & 7): sixteen rows read
+// at one logical chunk cover the 256-byte bank window.
+__device__ __forceinline__ int split_swz(int r, int c) { return c ^ ((r >> 1) & 7); }
+
+// This wave's loads of K bytes [k0, k0 + 128) of the tile's W and A rows into `dst` (W rows, then
+// A rows): each load brings 8 rows x 128 bytes.  Rows past the descriptors read 0.
+template <int I, int J>
+__device__ __forceinline__ void split_issue(__amdgpu_buffer_rsrc_t rw, __amdgpu_buffer_rsrc_t ra, uint8_t *__restrict__ dst,
+                                            const int (&lv)[2], int K, int k0) {
+#pragma unroll
+    for (int t = 0; t < 4 * I; ++t)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void *)(dst + t * 1024), 16,
+                                                 lv[t & 1], t * 8 * K + k0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 4 * J; ++t)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void *)(dst + (4 * I + t) * 1024), 16,
+                                                 lv[t & 1], t * 8 * K + k0, 0, 0);
+}
+
+__device__ __forceinline__ int32x8 split_frag(const uint8_t *__restrict__ rows, int r, int c) {
+    const uint4 lo = *reinterpret_cast<const uint4 *>(rows + r * kSplitBK + split_swz(r, c) * 16);
+    const uint4 hi = *reinterpret_cast<const uint4 *>(rows + r * kSplitBK + split_swz(r, c + 1) * 16);
+    return int32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+}
+
+// One chunk: refill `nxt` (read in the previous step), wait for `cur`, read its fragments, MFMAs.
+// The slots differ and are restrict-qualified: the reads of `cur` need not wait for the refill.
+template <bool kExact, int I, int J, int S>
+__device__ __forceinline__ void split_step(const uint8_t *__restrict__ cur, uint8_t *__restrict__ nxt, bool refill,
+                                           __amdgpu_buffer_rsrc_t rw, __amdgpu_buffer_rsrc_t ra, const int (&lv)[2], int K,
+                                           int k_next, bool second, int fr, int fc, floatx16 (&acc)[I][J]) {
+    constexpr int kLoads = 4 * (I + J);
+    wait_vm_fence<63>();  // the previous step's reads of `nxt` returned
+    if (refill) split_issue<I, J>(rw, ra, nxt, lv, K, k_next);
+    wait_vm_fence<(S - 1) * kLoads>();
+    SplitFrags<kExact, I, J> f;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+        for (int i = 0; i < I; ++i) f.w[kk][i] = split_frag(cur, 32 * i + fr, 4 * kk + fc);
+#pragma unroll
+        for (int j = 0; j < J; ++j) f.a[kk][j] = split_frag(cur + 32 * I * kSplitBK, 32 * j + fr, 4 * kk + fc);
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+        if (kk == 1 && !second) break;  // K % 128 == 64: the last chunk's second half lies past the row
+        if constexpr (kExact) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                half8_t wv[I], av[J];
+#pragma unroll
+                for (int i = 0; i < I; ++i) wv[i] = e4m3x8_to_f16(f.w[kk][i], c);
+#pragma unroll
+                for (int j = 0; j < J; ++j) av[j] = e4m3x8_to_f16(f.a[kk][j], c);
+#pragma unroll
+                for (int i = 0; i < I; ++i)
+#pragma unroll
+                    for (int j = 0; j < J; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wv[i], av[j], acc[i][j], 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < I; ++i)
+#pragma unroll
+                for (int j = 0; j < J; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.w[kk][i], f.a[kk][j], acc[i][j], 0, 0, 0, 0, 0, 0);
+        }
+    }
+}
+
+template <int I, int J, int NW, int S>
+constexpr int split_lds_bytes() {
+    const int ring = NW * S * 32 * (I + J) * kSplitBK, sums = NW * 32 * J * (32 * I + 4) * 4;
+    return ring > sums ? ring : sums;
+}
+
+template <bool kExact, int I, int J, int NW, int S>
+__global__ __launch_bounds__(64 * NW) void fp8_split_kernel(const uint8_t *__restrict__ A, const float *__restrict__ sa,
+                                                            const uint8_t *__restrict__ W, const float *__restrict__ sw,
+                                                            void *__restrict__ Y, int y_bf16, int y_vec, int M, int N, int K,
+                                                            int tiles_m, int tiles_n) {
+    constexpr int kBN = 32 * I, kBM = 32 * J, kStage = (kBN + kBM) * kSplitBK;
+    extern __shared__ __align__(16) uint8_t lds[];
+    // each XCD owns a contiguous run of tiles, in groups of up to 8 m tiles of one W panel (their A
+    // rows stay in the XCD's L2)
+    int pid = blockIdx.x;
+    {
+        const int per_xcd = tiles_m * tiles_n / kXcds, full = per_xcd * kXcds;
+        if (pid < full) pid = (pid % kXcds) * per_xcd + pid / kXcds;
+    }
+    const int span = 8 * tiles_n, first_m = pid / span * 8, gm = min(8, tiles_m - first_m);
+    const int m0 = (first_m + pid % span % gm) * kBM, n0 = pid % span / gm * kBN;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(W + static_cast<int64_t>(n0) * K), 0,
+                                                                        min(kBN, N - n0) * K, 0x00020000);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(A + static_cast<int64_t>(m0) * K), 0,
+                                                                        min(kBM, M - m0) * K, 0x00020000);
+    // lane i of a load writes LDS bytes [16 i, 16 i + 16): row i / 8, physical chunk i % 8
+    int lv[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) lv[u] = (lane >> 3) * K + split_swz(8 * u + (lane >> 3), lane & 7) * 16;
+    const int fr = lane & 31, fc = (lane >> 5) * 2;
+
+    floatx16 acc[I][J];
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+    // chunks of this wave; a chunk past its last one is neither loaded nor computed, and the waits
+    // of the steps that have no refill left are exact (they count down)
+    const int chunks = (K + kSplitBK - 1) / kSplitBK;
+    const int n_own = chunks > wave ? (chunks - wave + NW - 1) / NW : 0;
+    uint8_t *ring = lds + wave * S * kStage;
+    auto k_of = [&](int t) { return (wave + NW * t) * kSplitBK; };
+#pragma unroll
+    for (int t = 0; t < S; ++t)
+        if (t < n_own) split_issue<I, J>(rw, ra, ring + t * kStage, lv, K, k_of(t));
+    int t0 = 0;
+    for (; t0 + 2 * S - 2 < n_own; t0 += S)
+        static_for<S>([&](auto SI) {
+            constexpr int s = decltype(SI)::value;
+            split_step<kExact, I, J, S>(ring + s * kStage, ring + (s + S - 1) % S * kStage, t0 + s > 0, rw, ra, lv, K,
+                                        k_of(t0 + s + S - 1), true, fr, fc, acc);
+        });
+    for (; t0 < n_own; t0 += S)
+        static_for<S>([&](auto SI) {
+            constexpr int s = decltype(SI)::value;
+            const int t = t0 + s;
+            if (t < n_own) {
+                const bool refill = t > 0 && t + S - 1 < n_own;
+                const bool second = k_of(t) + 64 < K;
+                // chunks issued after chunk t: S - 1 of them, fewer at the end
+                if (t + S - 1 >= n_own) wait_vm_fence<0>();
+                split_step<kExact, I, J, S>(ring + s * kStage, ring + (s + S - 1) % S * kStage, refill, rw, ra, lv, K,
+                                            k_of(t + S - 1), second, fr, fc, acc);
+            }
+        });
+
+    // ---- sum of the waves' tiles: acc[i][j] reg 4 g + q holds n = 32 i + 8 g + 4 (lane / 32) + q,
+    // m = 32 j + lane % 32 ----
+    __syncthreads();  // every wave is done with its ring (all of its loads were waited for)
+    constexpr int kRow = kBN + 4;
+    float *sums = reinterpret_cast<float *>(lds);
+    static_for<J>([&](auto JJ) {
+        constexpr int j = decltype(JJ)::value;
+        static_for<I>([&](auto II) {
+            constexpr int i = decltype(II)::value;
+            static_for<4>([&](auto GG) {
+                constexpr int g = decltype(GG)::value;
+                *reinterpret_cast<float4 *>(sums + (wave * kBM + 32 * j + fr) * kRow + 32 * i + 8 * g + 2 * fc) =
+                    make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
+            });
+        });
+    });
+    __syncthreads();
+#pragma unroll
+    for (int o = threadIdx.x; o < kBM * kBN / 4; o += 64 * NW) {
+        const int ml = o / (kBN / 4), nl = o % (kBN / 4) * 4;
+        const int m = m0 + ml, n = n0 + nl;
+        if (m >= M || n >= N) continue;
+        float4 v = *reinterpret_cast<const float4 *>(sums + ml * kRow + nl);
+#pragma unroll
+        for (int w = 1; w < NW; ++w) {
+            const float4 p = *reinterpret_cast<const float4 *>(sums + (w * kBM + ml) * kRow + nl);
+            v.x += p.x, v.y += p.y, v.z += p.z, v.w += p.w;
+        }
+        const float am = sa[m];
+        float r[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) r[q] = n + q < N ? r[q] * am * sw[n + q] : 0.f;
+        const int64_t at = static_cast<int64_t>(m) * N + n;
+        if (y_vec) {  // N % 4 == 0 and Y 16-byte aligned
+            if (y_bf16)
+                *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(Y) + at) = make_uint2(f32x2_to_bf16x2_rne(r[0], r[1]), f32x2_to_bf16x2_rne(r[2], r[3]));
+            else
+                *reinterpret_cast<float4 *>(static_cast<float *>(Y) + at) = make_float4(r[0], r[1], r[2], r[3]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if (n + q < N) {
+                    if (y_bf16) static_cast<uint16_t *>(Y)[at + q] = f32_to_bf16_rne(r[q]);
+                    else static_cast<float *>(Y)[at + q] = r[q];
+                }
+            }
+        }
+    }
+}
+
 // Any shape (K % 4 == 0): one thread per output, exact e4m3 decode, f32 accumulation.
 __global__ void fp8_gemm_generic_kernel(const uint8_t *__restrict__ A, const float *__restrict__ sa,
                                         const uint8_t *__restrict__ W, const float *__restrict__ sw,
@@ -521,6 +740,38 @@ __global__ void fp8_gemm_generic_kernel(const uint8_t *__restrict__ A, const flo
 // devices (bit = device ordinal < 64) on which each variant's dynamic-LDS limit has been raised
 std::atomic<uint64_t> lds_attr_devices[2];
 
+// Raises a kernel's dynamic-LDS limit once per device (bit = device ordinal < 64).
+void raise_lds_limit(const void *kern, int bytes, std::atomic<uint64_t> &done) {
+    int dev = 0;
+    check_hip(hipGetDevice(&dev), "hipGetDevice");
+    const uint64_t bit = dev < 64 ? (uint64_t{1} << dev) : 0;
+    if (bit == 0 || !(done.load(std::memory_order_acquire) & bit)) {
+        check_hip(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "hipFuncSetAttribute(fp8)");
+        done.fetch_or(bit, std::memory_order_acq_rel);
+    }
+}
+
+int64_t cu_count() {
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+        return v;
+    return 256;
+}
+
+template <bool kExact, int I, int J, int NW, int S>
+void launch_split(const uint8_t *qa, const float *sa, int64_t m, const uint8_t *qw, const float *sw, int64_t n, int64_t k,
+                  void *y, int yb, hipStream_t st) {
+    constexpr int lds = split_lds_bytes<I, J, NW, S>();
+    static_assert(lds <= 160 * 1024, "LDS budget");
+    static std::atomic<uint64_t> attr_devices{0};
+    raise_lds_limit(reinterpret_cast<const void *>(&fp8_split_kernel<kExact, I, J, NW, S>), lds, attr_devices);
+    const int tiles_m = static_cast<int>((m + 32 * J - 1) / (32 * J)), tiles_n = static_cast<int>((n + 32 * I - 1) / (32 * I));
+    fp8_split_kernel<kExact, I, J, NW, S><<<dim3(tiles_m * tiles_n), dim3(64 * NW), lds, st>>>(
+        qa, sa, qw, sw, y, yb, (n % 4 == 0 && aligned(y, 16)) ? 1 : 0, static_cast<int>(m), static_cast<int>(n),
+        static_cast<int>(k), tiles_m, tiles_n);
+    check_launch("fp8_split");
+}
+
 int32_t gemm_fp8(const uint8_t *qa, const float *sa, int64_t m, const uint8_t *qw, const float *sw,
                  int64_t n, int64_t k, void *y, int32_t y_dtype, void *stream, char **out_error,
                  bool exact) {
@@ -535,17 +786,26 @@ int32_t gemm_fp8(const uint8_t *qa, const float *sa, int64_t m, const uint8_t *q
         // buffer resources address one 256-row panel: 256 * k bytes must fit in 31 bits
         const bool fast = k > 0 && k % BK == 0 && k < (1 << 23) && aligned(qa, 16) && aligned(qw, 16);
         if (fast) {
-            int dev = 0;
-            check_hip(hipGetDevice(&dev), "hipGetDevice");
-            const uint64_t bit = dev < 64 ? (uint64_t{1} << dev) : 0;
-            const auto kern = exact ? fp8_gemm_kernel<true> : fp8_gemm_kernel<false>;
-            std::atomic<uint64_t> &done = lds_attr_devices[exact ? 1 : 0];
-            if (bit == 0 || !(done.load(std::memory_order_acquire) & bit)) {
-                check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes),
-                          "hipFuncSetAttribute(fp8_gemm_kernel)");
-                done.fetch_or(bit, std::memory_order_acq_rel);
+            // K split over the waves (fp8_split_kernel) where the 256 x 256 tiles are few: 32 x 32
+            // tiles up to two per CU (11008 x 4096 at M = 64, 688 tiles: 15.5 us against 15.0 with
+            // 64 x 64), 64 x 64 up to 4 per CU (4096 x 4096 at M = 1024, 4.0 per CU: 42.1 us against
+            // 48.7 on 256 x 256; 11008 x 4096 at M = 512, 5.4: 56.2 against 50.1).  The exact form's
+            // 256 x 256 steps are twice as long: up to 6 (the same 5.4: 76.5 against 94.4; 4096 x
+            // 11008 at M = 2048, 8: 259 against 237).
+            const int64_t cus = cu_count();
+            const auto tiles = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t); };
+            if (tiles(32) <= 2 * cus) {
+                exact ? launch_split<true, 1, 1, 4, 2>(qa, sa, m, qw, sw, n, k, y, yb, st)
+                      : launch_split<false, 1, 1, 4, 2>(qa, sa, m, qw, sw, n, k, y, yb, st);
+                return;
             }
+            if (tiles(64) <= (exact ? 6 : 4) * cus) {
+                exact ? launch_split<true, 2, 2, 4, 2>(qa, sa, m, qw, sw, n, k, y, yb, st)
+                      : launch_split<false, 2, 2, 4, 2>(qa, sa, m, qw, sw, n, k, y, yb, st);
+                return;
+            }
+            const auto kern = exact ? fp8_gemm_kernel<true> : fp8_gemm_kernel<false>;
+            raise_lds_limit(reinterpret_cast<const void *>(kern), kLdsBytes, lds_attr_devices[exact ? 1 : 0]);
             const int tiles_m = static_cast<int>((m + BM - 1) / BM), tiles_n = static_cast<int>((n + BN - 1) / BN);
             kern<<<dim3(tiles_m * tiles_n), dim3(kThreads), kLdsBytes, st>>>(
                 qa, sa, qw, sw, y, yb,

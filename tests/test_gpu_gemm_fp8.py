@@ -81,6 +81,22 @@ def test_fp8_gemm_vs_oracle(cuda, m, n, k, exact):
         _check(y, qa_ref, sa_ref, qw_ref, sw_ref, exact, f"{m}x{n}x{k} {out}")
 
 
+# K split over waves: one half chunk (k = 64), an odd number of 64-wide halves, fewer chunks than
+# waves, many chunks; tile remainders in m and n.  The last three have more than two 32 x 32 tiles
+# per CU (64 x 64 tiles), the very last more than six 64 x 64 (256 x 256 tiles).
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 64), (31, 33, 192), (32, 32, 512), (33, 65, 576), (2, 200, 4160),
+                                   (520, 1050, 192), (545, 1024, 1088), (2500, 2900, 64)])
+def test_fp8_gemm_split_edges(cuda, m, n, k, exact):
+    a = synth.fp8_inputs(85, m, m, k)
+    w = synth.fp8_inputs(85, n, n, k) * np.float32(0.02)
+    qa, sa = ops.quantize_fp8(torch.from_numpy(a).to(cuda))
+    qw, sw = ops.quantize_fp8(torch.from_numpy(w).to(cuda))
+    for out in (torch.bfloat16, torch.float32):
+        y = ops.gemm_fp8(qa, sa, qw, sw, out_dtype=out, exact=exact)
+        _check(y, qa.cpu().numpy(), sa.cpu().numpy(), qw.cpu().numpy(), sw.cpu().numpy(), exact, f"{m}x{n}x{k} {out}")
+
+
 def _config4(cuda, m, n, k, seed):
     """both operands N(0, 1) with 0.5% of the elements x30; activations
     quantized per token from bf16, weights per output row from f32."""
