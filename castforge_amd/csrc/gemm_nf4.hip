@@ -255,7 +255,9 @@ void nf4_mfma_kernel(Nf4Batch b) {
         static_for<kWDepth - kStages>([&](auto I) { wload(wr[decltype(I)::value], chunk_of(decltype(I)::value)); });
         static_for<kStages - 1>([&](auto I) {
             constexpr int t = decltype(I)::value;
+            asm volatile("" ::: "memory");
             issue(RC, ring + t * kStage, chunk_of(t));
+            asm volatile("" ::: "memory");
             wload(wr[t + kWDepth - kStages], chunk_of(t + kWDepth - kStages));
         });
         // Step t runs chunk t's MFMAs from operands decoded in step t - 1 and, between them, folds
@@ -280,14 +282,18 @@ void nf4_mfma_kernel(Nf4Batch b) {
                         auto I, int t) __attribute__((always_inline)) {
             constexpr int i = decltype(I)::value;
             issue(RC, nxt, chunk_of(t + kStages - 1));
+            asm volatile("" ::: "memory");  // the waits count the code loads after the x loads
             wload(wr[(i + kWDepth - 1) % kWDepth], chunk_of(t + kWDepth - 1));
             mma(cur, dec[i & 1], part[i & 1]);
             fold(dec[(i + 1) & 1].am, part[(i + 1) & 1]);
             decode(lut, wr[(i + 1) % kWDepth], am_of(t + 1, wr[(i + 1) % kWDepth]), dec[(i + 1) & 1]);
         };
-        auto step = [&](auto I, int t) {
+        // Steps of a whole unrolled group wait by count; the last, partial group waits for everything:
+        // there the compiler drops the code and absmax loads that no later step consumes, so fewer loads
+        // follow chunk t's x than the count allows (K = 2048 has read x stages before they landed).
+        auto step = [&](auto whole, auto I, int t) {
             constexpr int i = decltype(I)::value;  // t modulo kWDepth (a multiple of kStages and of 2)
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm(kPer + 2) & ~(15 << 8));
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(decltype(whole)::value ? kPer + 2 : 0) & ~(15 << 8));
             // unconditional: the compiler's own wait tracking then sees every LDS read retired
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(63) & ~(15 << 8));
             __builtin_amdgcn_s_barrier();
@@ -296,9 +302,9 @@ void nf4_mfma_kernel(Nf4Batch b) {
         static_assert(kWDepth % kStages == 0 && kWDepth % 2 == 0, "one unrolled group covers every ring");
         int t = 0;
         for (; t + kWDepth <= steps; t += kWDepth)
-            static_for<kWDepth>([&](auto I) { step(I, t + decltype(I)::value); });
+            static_for<kWDepth>([&](auto I) { step(std::true_type{}, I, t + decltype(I)::value); });
         static_for<kWDepth>([&](auto I) {
-            if (t + decltype(I)::value < steps) step(I, t + decltype(I)::value);
+            if (t + decltype(I)::value < steps) step(std::false_type{}, I, t + decltype(I)::value);
         });
         // the last chunk's partial: part[(steps - 1) & 1], its absmax in dec[(steps - 1) & 1]
         if ((steps - 1) & 1) fold(dec[1].am, part[1]);

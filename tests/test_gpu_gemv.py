@@ -188,6 +188,26 @@ def test_batched_mid_m(cuda, fmt, m):
         _close(y1, ref)
 
 
+@pytest.mark.parametrize("m", [17, 40])
+@pytest.mark.parametrize("steps", [2, 3, 4, 5, 6, 9, 11])
+def test_nf4_partial_step_groups(cuda, steps, m):
+    """NF4 at M > 16 with every remainder of the K loop's groups of six 64-wide steps per K part (two
+    parts up to K = 6144), on weights no earlier call has brought into the caches: against float64."""
+    n, k = 1500, 128 * steps
+    w = torch.from_numpy(synth.weight(740 + steps, 1, n, k)).to(cuda)
+    _, x = _x(750 + steps, m, k, cuda)
+    p = ops.quantize_nf4(w, 64)
+    wd = ops.dequantize_nf4(p).cpu().double()
+    x64 = x.cpu().double()
+    torch.empty(1 << 28, dtype=torch.uint8, device=cuda).zero_()  # 256 MB through the caches
+    y = ops.gemm_nf4(x, p, torch.float32).cpu().double()
+    mag = x64.abs() @ wd.abs().t()
+    # T_hi + T_lo is within 2^-17 of T, the dequantized weight within 2^-24; f32 sums: one rounding an
+    # MFMA step of 16, a scale every 64, the K parts
+    bound = (2.0 ** -17 + (k / 8 + k / 64 + 4) * 2.0 ** -24) * mag
+    assert bool(((y - x64 @ wd.t()).abs() <= bound).all())
+
+
 def test_nf4_batched_rejects_mixed_blocks(cuda):
     ps = [ops.quantize_nf4(torch.zeros((16, 256), device=cuda), b) for b in (64, 32)]
     xs = [torch.zeros((1, 256), dtype=torch.bfloat16, device=cuda)] * 2
