@@ -1,4 +1,5 @@
 // Library-level C-ABI entry points: version, string ownership, device description.
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <string>
@@ -14,6 +15,16 @@ char *dup_string(const std::string &s) {
     for (size_t i = 0; i < s.size(); ++i) p[i] = (s[i] == '\0') ? ' ' : s[i];  // ffi.rs:210
     p[s.size()] = '\0';
     return p;
+}
+
+int64_t cu_count() {
+    static std::atomic<int> cus[64];
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 256;
+    if (dev < 64 && (v = cus[dev].load(std::memory_order_relaxed)) > 0) return v;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) return 256;
+    if (dev < 64) cus[dev].store(v, std::memory_order_relaxed);
+    return v;
 }
 
 }  // namespace cfh

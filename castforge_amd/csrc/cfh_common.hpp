@@ -42,6 +42,9 @@ inline void check_hip(hipError_t e, const char *what) {
 // objects, or an earlier asynchronous fault).
 inline void check_launch(const char *kernel) { check_hip(hipGetLastError(), kernel); }
 
+// Compute units of the current device (asked once per device).
+int64_t cu_count();
+
 inline bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
 
 // Runs `body` and turns every outcome into the reference's status codes.

@@ -649,13 +649,16 @@ __global__ __launch_bounds__(64 * NW) void fp8_split_kernel(const uint8_t *__res
     uint8_t *ring = lds + wave * S * kStage;
     auto k_of = [&](int t) { return (wave + NW * t) * kSplitBK; };
 #pragma unroll
-    for (int t = 0; t < S; ++t)
-        if (t < n_own) split_issue<I, J>(rw, ra, ring + t * kStage, lv, K, k_of(t));
+    for (int t = 0; t < S - 1; ++t)
+        if (t < n_own) {
+            asm volatile("" ::: "memory");  // the waits count whole chunks
+            split_issue<I, J>(rw, ra, ring + t * kStage, lv, K, k_of(t));
+        }
     int t0 = 0;
     for (; t0 + 2 * S - 2 < n_own; t0 += S)
         static_for<S>([&](auto SI) {
             constexpr int s = decltype(SI)::value;
-            split_step<kExact, I, J, S>(ring + s * kStage, ring + (s + S - 1) % S * kStage, t0 + s > 0, rw, ra, lv, K,
+            split_step<kExact, I, J, S>(ring + s * kStage, ring + (s + S - 1) % S * kStage, true, rw, ra, lv, K,
                                         k_of(t0 + s + S - 1), true, fr, fc, acc);
         });
     for (; t0 < n_own; t0 += S)
@@ -663,7 +666,7 @@ __global__ __launch_bounds__(64 * NW) void fp8_split_kernel(const uint8_t *__res
             constexpr int s = decltype(SI)::value;
             const int t = t0 + s;
             if (t < n_own) {
-                const bool refill = t > 0 && t + S - 1 < n_own;
+                const bool refill = t + S - 1 < n_own;
                 const bool second = k_of(t) + 64 < K;
                 // chunks issued after chunk t: S - 1 of them, fewer at the end
                 if (t + S - 1 >= n_own) wait_vm_fence<0>();
@@ -749,13 +752,6 @@ void raise_lds_limit(const void *kern, int bytes, std::atomic<uint64_t> &done) {
         check_hip(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes), "hipFuncSetAttribute(fp8)");
         done.fetch_or(bit, std::memory_order_acq_rel);
     }
-}
-
-int64_t cu_count() {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-        return v;
-    return 256;
 }
 
 template <bool kExact, int I, int J, int NW, int S>

@@ -996,19 +996,14 @@ int pick_tile(int64_t M, int64_t N) {
             if (std::strcmp(e, name) == 0) return t;
         }
     }
-    int cus = 256;
-    int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        int v = 0;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) cus = v;
-    }
+    const int64_t cus = cu_count();
     // 128 x 256 and 64 x 128 are left to the override: at every shape measured they lost to
     // the next smaller square tile (W_gate / W_down of the 7B block at M = 512 / 1024 / 4096,
     // NF4 / Q8_0 / INT8: e.g. Q8_0 11008 x 4096 at M = 1024 406 against 278 us on 128 x 128,
     // NF4 4096 x 11008 at M = 512 254 on 64 x 128 against 196 us on 64 x 64)
     for (int t : {PF_256x256, PF_128x128, PF_64x64}) {
         const int64_t tiles = ((M + kPfTileM[t] - 1) / kPfTileM[t]) * ((N + kPfTileN[t] - 1) / kPfTileN[t]);
-        if (M > kPfTileM[t] / 2 && tiles >= static_cast<int64_t>(cus)) return t;
+        if (M > kPfTileM[t] / 2 && tiles >= cus) return t;
     }
     return PF_64x64;
 }
@@ -1043,18 +1038,14 @@ bool i4_eligible(const PfArgs &a, int fmt) {
         if (std::strcmp(e, "0") == 0) return false;
         if (std::strcmp(e, "1") == 0) return true;
     }
-    int cus = 256, dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        int v = 0;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) cus = v;
-    }
+    const int64_t cus = cu_count();
     const int64_t tiles = ((a.M + 127) / 128) * static_cast<int64_t>((a.N + kI4BN - 1) / kI4BN);
     // INT4: one tile per 6 CUs.  The GGUF forms fold every two MFMA steps and INT8's generic
     // kernel is already one term, so they switch later (measured on 256 CUs, us generic / one-
     // MFMA): Q4_0 / Q8_0 11008 x 4096 at M = 128 (43 tiles) 65 / 76 and 75 / 92, at M = 256
     // (86) 102 / 77 and 116 / 92; INT8 4096 x 11008 and 4096 x 4096 at M = 1024 (128 tiles)
     // 124 / 136 and 51 / 55, 11008 x 4096 at M = 512 (172) 73 / 56.
-    if (fmt == FMT_INT8) return 8 * tiles >= 5 * static_cast<int64_t>(cus);
+    if (fmt == FMT_INT8) return 8 * tiles >= 5 * cus;
     if (fmt == FMT_Q4G || fmt == FMT_Q8G || fmt == FMT_I4G32 || fmt == FMT_I4G64) return 3 * tiles >= cus;
     return 6 * tiles >= cus;
 }

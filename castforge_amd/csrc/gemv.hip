@@ -1629,6 +1629,38 @@ bool prefill_try(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, in
                  const void *codes, const void *scales, const uint32_t *zeros, int per_row, void *y,
                  int y_bf16, hipStream_t st);
 
+// K split over a workgroup's waves (gemm_split.hip); false where it does not take the problem.
+bool qsplit_try(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes,
+                const void *scales, const uint32_t *zeros, int per_row, void *y, int y_bf16, hipStream_t st);
+bool qsplit_ok(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes, const void *scales);
+void qsplit_batch(int fmt, int64_t m, int count, const uint16_t *const *x, const int64_t *n, const int64_t *k,
+                  const int64_t *group, const void *const *codes, const void *const *scales, const uint32_t *const *zeros,
+                  const int *per_row, void *const *y, int y_bf16, hipStream_t st);
+
+// A batch (each problem passes skinny_ok): the problems that qsplit_kernel takes in one launch of
+// it, as single calls do, the others in one launch of the skinny kernels.
+void launch_batch(int fmt, Problem *ps, int count, int64_t m, int y_bf16, hipStream_t st) {
+    const uint16_t *x[kMaxProblems];
+    int64_t n[kMaxProblems], k[kMaxProblems], group[kMaxProblems];
+    const void *codes[kMaxProblems], *scales[kMaxProblems];
+    const uint32_t *zeros[kMaxProblems];
+    int per_row[kMaxProblems];
+    void *y[kMaxProblems];
+    int used = 0, rest = 0;
+    for (int i = 0; i < count; ++i) {
+        const Problem p = ps[i];
+        if (!qsplit_ok(fmt, p.x, m, p.n, p.k, p.group, p.codes, p.scales)) {
+            ps[rest++] = p;
+            continue;
+        }
+        x[used] = p.x, n[used] = p.n, k[used] = p.k, group[used] = p.group, codes[used] = p.codes, scales[used] = p.scales;
+        zeros[used] = p.zeros, per_row[used] = p.scale_per_row, y[used] = p.y;
+        ++used;
+    }
+    if (used) qsplit_batch(fmt, m, used, x, n, k, group, codes, scales, zeros, per_row, y, y_bf16, st);
+    if (rest) launch_skinny(fmt, ps, rest, m, y_bf16, st);
+}
+
 // Largest M a single problem runs on the skinny kernels; beyond it the prefill kernel is
 // faster (measured on W_gate / W_up / W_down of a 7B block: INT8 and Q4_0 at M = 48 / 64 take
 // 138 / 149 and 309 / 323 us there against 103 / 100 and 200 / 197 us on the prefill kernel;
@@ -1674,7 +1706,8 @@ int32_t castforge_hip_gemv_w4a16(const uint16_t *x, int64_t m, int64_t n, int64_
         require(k == 0 || (scales_f16 && zeros), "scales and zeros must not be NULL");
         hipStream_t st = static_cast<hipStream_t>(stream);
         const int yb = y_dtype == CFH_DTYPE_BF16;
-        if (!gemv_try_skinny(FMT_INT4, x, m, n, k, group, codes, scales_f16, zeros, 1, y, yb, st) &&
+        if (!qsplit_try(FMT_INT4, x, m, n, k, group, codes, scales_f16, zeros, 1, y, yb, st) &&
+            !gemv_try_skinny(FMT_INT4, x, m, n, k, group, codes, scales_f16, zeros, 1, y, yb, st) &&
             !prefill_try(FMT_INT4, x, m, n, k, group, codes, scales_f16, zeros, 1, y, yb, st))
             gemv_generic(FMT_INT4, x, m, n, k, group, codes, scales_f16, zeros, 1, y, yb, st);
     });
@@ -1691,7 +1724,8 @@ int32_t castforge_hip_gemv_w8a16(const uint16_t *x, int64_t m, int64_t n, int64_
         require(scales != nullptr, "scales must not be NULL");
         hipStream_t st = static_cast<hipStream_t>(stream);
         const int yb = y_dtype == CFH_DTYPE_BF16, pr = granularity == CFH_GRAN_CHANNEL;
-        if (!gemv_try_skinny(FMT_INT8, x, m, n, k, 0, codes, scales, nullptr, pr, y, yb, st) &&
+        if (!qsplit_try(FMT_INT8, x, m, n, k, 0, codes, scales, nullptr, pr, y, yb, st) &&
+            !gemv_try_skinny(FMT_INT8, x, m, n, k, 0, codes, scales, nullptr, pr, y, yb, st) &&
             !prefill_try(FMT_INT8, x, m, n, k, 0, codes, scales, nullptr, pr, y, yb, st))
             gemv_generic(FMT_INT8, x, m, n, k, 0, codes, scales, nullptr, pr, y, yb, st);
     });
@@ -1744,6 +1778,7 @@ int32_t castforge_hip_gemv_gguf(int32_t ggml_type, const uint16_t *x, int64_t m,
             launch_skinny(fmt, ps, 2, 1, yb, st);
             return;
         }
+        if (qsplit_try(fmt, x, m, n, k, 32, codes, scales_f16, nullptr, 1, y, yb, st)) return;
         // split-K kernel at M = 1, the skinny kernel (x read per wave) beyond
         if (gemv_try_skinny(fmt, x, m, n, k, 32, codes, scales_f16, nullptr, 1, y, yb, st)) return;
         // larger M: the prefill MFMA kernel reads the planes directly
@@ -1775,7 +1810,7 @@ int32_t castforge_hip_gemv_gguf_batched(int32_t ggml_type, const cfh_gguf_proble
                     "and 16-byte aligned x / codes / scales");
             ps[used++] = p;
         }
-        if (used) launch_skinny(fmt, ps, used, m, y_dtype == CFH_DTYPE_BF16, static_cast<hipStream_t>(stream));
+        if (used) launch_batch(fmt, ps, used, m, y_dtype == CFH_DTYPE_BF16, static_cast<hipStream_t>(stream));
     });
 }
 
@@ -1800,7 +1835,7 @@ int32_t castforge_hip_gemv_w4a16_batched(const cfh_w4a16_problem_t *problems, in
                     "batched GEMV needs k % 128 == 0, group % 128 == 0 and 16-byte aligned x/codes");
             ps[used++] = p;
         }
-        if (used) launch_skinny(FMT_INT4, ps, used, m, y_dtype == CFH_DTYPE_BF16,
+        if (used) launch_batch(FMT_INT4, ps, used, m, y_dtype == CFH_DTYPE_BF16,
                                 static_cast<hipStream_t>(stream));
     });
 }
@@ -1827,7 +1862,7 @@ int32_t castforge_hip_gemv_w8a16_batched(const cfh_w8a16_problem_t *problems, in
             require(skinny_ok(FMT_INT8, p, m), "batched GEMV needs k % 64 == 0 and 16-byte aligned x/codes");
             ps[used++] = p;
         }
-        if (used) launch_skinny(FMT_INT8, ps, used, m, y_dtype == CFH_DTYPE_BF16, static_cast<hipStream_t>(stream));
+        if (used) launch_batch(FMT_INT8, ps, used, m, y_dtype == CFH_DTYPE_BF16, static_cast<hipStream_t>(stream));
     });
 }
 

@@ -1,0 +1,55 @@
+"""GPU parity of the K-split MFMA kernel (M >= 2, small and mid-sized) against float64 products of
+the dequantized weights, at sizes that reach each of its tiles and their remainders."""
+import numpy as np
+import pytest
+import torch
+
+from castforge_amd import ffi, ops, synth
+
+pytestmark = pytest.mark.gpu
+
+# (m, n): 32 x 32 tiles (M <= 32; few tiles); 32 (n) x 64 (M <= 64, M > 64); 64 x 64 (M <= 64,
+# M > 64); 64 (n) x 128; one row and column past or short of a tile
+SHAPES = [(2, 1), (31, 65), (33, 64), (64, 97), (40, 4200), (70, 2803), (40, 9000), (130, 4000), (300, 3301)]
+
+
+def _weight(fmt, n, k, cuda):
+    w = torch.from_numpy(synth.weight(31, n, n, k)).to(cuda)
+    if fmt.startswith("int4"):
+        p = ops.quantize_int4g(w, int(fmt[5:]))
+        return ops.dequantize_int4g(p), lambda x, o: ops.gemm_w4a16(x, p, o), lambda x, y: ops.gemv_w4a16_batched([x], [p], [y])
+    if fmt.startswith("int8"):
+        gran = fmt[5:]
+        q, s = ops.quantize_int8(w, 8, gran)
+        return (ops.dequantize_int8(q, s, gran), lambda x, o: ops.gemm_w8a16(x, q, s, gran, o),
+                lambda x, y: ops.gemv_w8a16_batched([x], [(q, s)], [y], gran))
+    ty, size = (ffi.GGML_Q4_0, 18) if fmt == "q4_0" else (ffi.GGML_Q8_0, 34)
+    rng = np.random.default_rng(n + k)
+    raw = rng.integers(0, 256, (n * k // 32, size), dtype=np.uint8)
+    raw[:, :2] = rng.uniform(1e-3, 2e-3, (n * k // 32, 1)).astype(np.float16).view(np.uint8)
+    p = ops.gguf_repack(ty, torch.from_numpy(raw.reshape(-1)).to(cuda), n, k)
+    return ops.dequantize_gguf(p), lambda x, o: ops.gemm_gguf(x, p, o), lambda x, y: ops.gemv_gguf_batched([x], [p], [y])
+
+
+# k: fewer 64-wide chunks than the workgroup's eight waves, and 18 chunks (some waves one more)
+@pytest.mark.parametrize("fmt,k", [("int4_32", 192), ("int4_64", 192), ("int4_64", 1152), ("int4_128", 1152),
+                                   ("int4_256", 1280), ("int8_channel", 192), ("int8_tensor", 1152),
+                                   ("q4_0", 1152), ("q8_0", 192), ("q8_0", 1152)])
+@pytest.mark.parametrize("m,n", SHAPES)
+def test_split_vs_float64(cuda, fmt, k, m, n):
+    wd, run, run_batched = _weight(fmt, n, k, cuda)
+    x = torch.from_numpy(synth.activations_bf16(33, m, m, k).view(np.int16)).view(torch.bfloat16).to(cuda)
+    x64, w64 = x.cpu().double(), wd.cpu().double()
+    ref, mag = x64 @ w64.t(), x64.abs() @ w64.abs().t()
+    # f32 roundings on a path of one product: an MFMA step every 16 of K, a scale every 32, the sum of
+    # eight waves and the dequantized weight's own; each at most 2^-24 of the magnitudes summed
+    bound = (k / 16 + k / 32 + 10) * 2.0 ** -24 * mag
+    y = run(x, torch.float32)
+    assert bool(((y.cpu().double() - ref).abs() <= bound).all()), (fmt, m, n, k)
+    yb = run(x, torch.bfloat16)
+    assert torch.equal(yb, y.to(torch.bfloat16))
+    # (batched INT4 takes groups of 128; a single GGUF call of two rows runs the M = 1 kernel)
+    if m <= 64 and fmt in ("int4_128", "int8_channel", "int8_tensor") or 2 < m <= 64 and fmt[0] == "q":
+        yy = torch.empty_like(y)
+        run_batched(x, yy)
+        assert torch.equal(yy, y)
