@@ -1435,20 +1435,6 @@ __global__ void q40_from_planes_kernel(const uint8_t *pc, const uint16_t *pd, in
 }
 
 // ---- host ----------------------------------------------------------------------------------
-int cu_count() {
-    static std::mutex mu;
-    static std::map<int, int> cache;
-    int dev = 0;
-    check_hip(hipGetDevice(&dev), "hipGetDevice");
-    std::lock_guard<std::mutex> g(mu);
-    auto it = cache.find(dev);
-    if (it != cache.end()) return it->second;
-    int cus = 0;
-    check_hip(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "hipDeviceGetAttribute");
-    cache[dev] = cus;
-    return cus;
-}
-
 // Workgroups per problem in proportion to its code bytes (largest remainders; at least one per
 // problem, at most one per 8-row unit): every CU then streams about the same number of bytes.
 std::vector<int> workgroups_per_problem(const std::vector<int64_t> &bytes, const std::vector<int64_t> &units,
@@ -1642,7 +1628,7 @@ void planes_xr_launch(const cfh_w4a16_problem_t *problems, int32_t count, int64_
         xcost.push_back(static_cast<int64_t>(c * static_cast<double>(m * problems[i].k)));
         lo_wgs.push_back(std::max<int64_t>(1, (units[static_cast<size_t>(i)] + 2 * (max_tiles - 1) - 1) / (2 * (max_tiles - 1))));
     }
-    std::vector<int> wgs = workgroups_balanced(bytes, xcost, lo_wgs, units, cu_count() * kWgPerCu);
+    std::vector<int> wgs = workgroups_balanced(bytes, xcost, lo_wgs, units, static_cast<int>(cu_count()) * kWgPerCu);
     PBatch<CFH_MAX_BATCH> b{};
     int64_t lds = 0, grid = 0;
     for (int j = 0; j < count; ++j) {
@@ -1701,7 +1687,7 @@ void planes_batched(const cfh_w4a16_problem_t *problems, int32_t count, int64_t 
     require(m >= 1 && m <= 16, "the GEMV planes kernels take M = 1..16");
     require(y_dtype == CFH_DTYPE_F32 || y_dtype == CFH_DTYPE_BF16, "y_dtype must be F32 or BF16");
     const int mr = m == 1 ? 1 : 4;
-    const int W = cu_count() * kWgPerCu;
+    const int W = static_cast<int>(cu_count()) * kWgPerCu;
     for (int i = 0; i < count; ++i) {
         const cfh_w4a16_problem_t &q = problems[i];
         require(q.group == kGroup, "GEMV planes hold INT4 groups of 128");
@@ -1863,7 +1849,7 @@ void nf4_planes_batched(const cfh_nf4_problem_t *problems, int32_t count, int64_
     const int64_t block = problems[0].block;
     require(nf4_block_ok(block), "NF4 block must be a power of two >= 32");
     const int64_t nbpc = block >= kGroup ? 1 : kGroup / block;
-    const int W = cu_count();
+    const int W = static_cast<int>(cu_count());
     std::vector<int64_t> bytes, units;
     for (int i = 0; i < count; ++i) {
         const cfh_nf4_problem_t &q = problems[i];
@@ -1917,7 +1903,7 @@ void q40_planes_batched(const cfh_gguf_problem_t *problems, int32_t count, int64
     require(problems != nullptr, "problems must not be NULL");
     require(m == 1, "the Q4_0 planes kernel takes M = 1");
     require(y_dtype == CFH_DTYPE_F32 || y_dtype == CFH_DTYPE_BF16, "y_dtype must be F32 or BF16");
-    const int W = cu_count();
+    const int W = static_cast<int>(cu_count());
     std::vector<int64_t> bytes, units;
     for (int i = 0; i < count; ++i) {
         const cfh_gguf_problem_t &q = problems[i];
