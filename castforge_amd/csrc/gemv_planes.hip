@@ -1524,7 +1524,7 @@ std::vector<int> workgroups_balanced(const std::vector<int64_t> &bytes, const st
     };
     double lo = fmax, hi = fmax + 1.0;
     for (int it = 0; it < 200 && total(hi) > W; ++it) hi = fmax + 2.0 * (hi - fmax);
-    for (int it = 0; it < 100; ++it) {
+    for (int it = 0; it < 100 && hi - lo > 1e-9 * hi; ++it) {  // shares are whole workgroups
         const double mid = 0.5 * (lo + hi);
         if (mid <= fmax || total(mid) > W) lo = mid;
         else hi = mid;

@@ -10,6 +10,7 @@ from __future__ import annotations
 import ctypes
 import os
 import re
+import threading
 from ctypes import POINTER, c_char_p, c_int32, c_int64, c_uint16, c_uint32, c_uint8, c_void_p
 from pathlib import Path
 
@@ -183,11 +184,26 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+class _ThreadError(threading.local):
+    """A thread's out_error slot (every entry point clears it on entry)."""
+
+    def __init__(self):
+        self.value = c_char_p()
+        self.ref = ctypes.byref(self.value)
+
+
+_error = _ThreadError()
+_functions = {}  # entry points by name, bound once
+
+
 def call(name: str, *args) -> None:
     """Calls an entry point that ends with `char** out_error` and raises on non-zero status."""
-    err = c_char_p()
-    rc = getattr(lib(), name)(*args, ctypes.byref(err))
+    fn = _functions.get(name)
+    if fn is None:
+        fn = _functions[name] = getattr(lib(), name)
+    rc = fn(*args, _error.ref)
     if rc != 0:
+        err = _error.value
         msg = err.value.decode("utf-8", "replace") if err.value else "(no message)"
         if err.value is not None:
             lib().castforge_hip_free_string(ctypes.cast(err, c_void_p))

@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import struct
 from dataclasses import dataclass
 
 import torch
@@ -21,7 +22,13 @@ def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# the raw hipStream_t of the device's current stream, without a Stream object around it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t: torch.Tensor) -> int:
+    if _raw_stream is not None and t.is_cuda:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
@@ -243,17 +250,26 @@ def _check_batch(xs: list[torch.Tensor], ys: list[torch.Tensor], m: int, ns: lis
     """Validates the activations and preallocated outputs of a batched launch: every x bf16
     [m, k] and every y contiguous [m, n] on x's device, all y of ONE dtype (f32 or bf16, the
     C ABI takes a single y_dtype for the batch).  Returns that dtype's ABI code."""
-    dev = xs[0].device
+    dev, yt = xs[0].get_device(), ys[0].dtype
+    seen = seen_k = None
     for x, y, n, k in zip(xs, ys, ns, ks):
-        _check_x(x, k)
+        if x is not seen or k != seen_k:  # q / k / v share one x: checked once per call
+            _check_x(x, k)
+            seen, seen_k = x, k
         _dev(y)
-        if x.device != dev or y.device != dev:
+        if x.get_device() != dev or y.get_device() != dev:
             raise ValueError("every x and y of a batch must be on the same device")
-        if x.shape[0] != m or tuple(y.shape) != (m, n):
+        if x.shape[0] != m or y.shape != (m, n):
             raise ValueError("all problems must share M and y must be [M, n]")
-        if y.dtype != ys[0].dtype:
+        if y.dtype != yt:
             raise ValueError(f"every y of a batch must have one dtype: {ys[0].dtype} and {y.dtype}")
     return _out_dtype(ys[0].dtype)
+
+
+def _problem_array(cls, words: list[int]):
+    """A ctypes array of `cls` (a structure of 8-byte fields) from its fields in order."""
+    n = len(words) * 8 // ctypes.sizeof(cls)
+    return (cls * n).from_buffer(bytearray(struct.pack(f"{len(words)}q", *words)))
 
 
 def gemm_w4a16(x: torch.Tensor, p: Int4Packed, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
@@ -316,10 +332,10 @@ def gemv_w4a16_batched(xs: list[torch.Tensor], ps: list[Int4Packed], ys: list[to
         return
     m = xs[0].shape[0]
     yd = _check_batch(xs, ys, m, [p.n for p in ps], [p.k for p in ps])
-    arr = (ffi.W4A16Problem * len(ps))()
-    for i, (x, p, y) in enumerate(zip(xs, ps, ys)):
-        arr[i] = ffi.W4A16Problem(_ptr(x), _ptr(p.codes), _ptr(p.scales), _ptr(p.zeros), _ptr(y),
-                                  p.n, p.k, p.group)
+    words = []
+    for x, p, y in zip(xs, ps, ys):
+        words += (x.data_ptr(), p.codes.data_ptr(), p.scales.data_ptr(), p.zeros.data_ptr(), y.data_ptr(), p.n, p.k, p.group)
+    arr = _problem_array(ffi.W4A16Problem, words)
     ffi.call("castforge_hip_gemv_w4a16_batched", arr, len(ps), m, yd, _stream(xs[0]))
 
 
@@ -374,9 +390,10 @@ def gemv_w4a16_planes_batched(xs: list[torch.Tensor], ps: list[Int4Planes], ys: 
     if not 1 <= m <= 16:
         raise ValueError("the GEMV planes kernels take x of 1..16 rows")
     yd = _check_batch(xs, ys, m, [p.n for p in ps], [p.k for p in ps])
-    arr = (ffi.W4A16Problem * len(ps))()
-    for i, (x, p, y) in enumerate(zip(xs, ps, ys)):
-        arr[i] = ffi.W4A16Problem(_ptr(x), _ptr(p.codes), _ptr(p.scales), _ptr(p.zeros), _ptr(y), p.n, p.k, 128)
+    words = []
+    for x, p, y in zip(xs, ps, ys):
+        words += (x.data_ptr(), p.codes.data_ptr(), p.scales.data_ptr(), p.zeros.data_ptr(), y.data_ptr(), p.n, p.k, 128)
+    arr = _problem_array(ffi.W4A16Problem, words)
     ffi.call("castforge_hip_gemv_w4a16_planes_batched", arr, len(ps), m, yd, _stream(xs[0]))
 
 
@@ -411,9 +428,10 @@ def gemv_nf4_batched(xs: list[torch.Tensor], ps: list["Nf4Packed"], ys: list[tor
         return
     m = xs[0].shape[0]
     yd = _check_batch(xs, ys, m, [p.n for p in ps], [p.k for p in ps])
-    arr = (ffi.Nf4Problem * len(ps))()
-    for i, (x, p, y) in enumerate(zip(xs, ps, ys)):
-        arr[i] = ffi.Nf4Problem(_ptr(x), _ptr(p.codes), _ptr(p.absmax), _ptr(y), p.n, p.k, p.block)
+    words = []
+    for x, p, y in zip(xs, ps, ys):
+        words += (x.data_ptr(), p.codes.data_ptr(), p.absmax.data_ptr(), y.data_ptr(), p.n, p.k, p.block)
+    arr = _problem_array(ffi.Nf4Problem, words)
     ffi.call("castforge_hip_gemv_nf4_batched", arr, len(ps), m, yd, _stream(xs[0]))
 
 
@@ -470,9 +488,10 @@ def gemv_nf4_planes_batched(xs: list[torch.Tensor], ps: list[Nf4Planes], ys: lis
     if m != 1:
         raise ValueError("the NF4 planes kernel takes x of one row")
     yd = _check_batch(xs, ys, m, [p.n for p in ps], [p.k for p in ps])
-    arr = (ffi.Nf4Problem * len(ps))()
-    for i, (x, p, y) in enumerate(zip(xs, ps, ys)):
-        arr[i] = ffi.Nf4Problem(_ptr(x), _ptr(p.codes), _ptr(p.absmax), _ptr(y), p.n, p.k, p.block)
+    words = []
+    for x, p, y in zip(xs, ps, ys):
+        words += (x.data_ptr(), p.codes.data_ptr(), p.absmax.data_ptr(), y.data_ptr(), p.n, p.k, p.block)
+    arr = _problem_array(ffi.Nf4Problem, words)
     ffi.call("castforge_hip_gemv_nf4_planes_batched", arr, len(ps), m, yd, _stream(xs[0]))
 
 
@@ -665,9 +684,10 @@ def gemv_gguf_batched(xs: list[torch.Tensor], ps: list[GgufPacked], ys: list[tor
     if any(p.ggml_type != t for p in ps):
         raise ValueError("problems must share the GGML type and M, with x [M, k] and y [M, n]")
     yd = _check_batch(xs, ys, m, [p.n for p in ps], [p.k for p in ps])
-    arr = (ffi.GgufProblem * len(ps))()
-    for i, (x, p, y) in enumerate(zip(xs, ps, ys)):
-        arr[i] = ffi.GgufProblem(_ptr(x), _ptr(p.codes), _ptr(p.scales), _ptr(y), p.n, p.k)
+    words = []
+    for x, p, y in zip(xs, ps, ys):
+        words += (x.data_ptr(), p.codes.data_ptr(), p.scales.data_ptr(), y.data_ptr(), p.n, p.k)
+    arr = _problem_array(ffi.GgufProblem, words)
     ffi.call("castforge_hip_gemv_gguf_batched", t, arr, len(ps), m, yd, _stream(xs[0]))
 
 
@@ -718,9 +738,10 @@ def gemv_gguf_q4_0_planes_batched(xs: list[torch.Tensor], ps: list[Q40Planes], y
     if m != 1:
         raise ValueError("the Q4_0 planes kernel takes x of one row")
     yd = _check_batch(xs, ys, m, [p.n for p in ps], [p.k for p in ps])
-    arr = (ffi.GgufProblem * len(ps))()
-    for i, (x, p, y) in enumerate(zip(xs, ps, ys)):
-        arr[i] = ffi.GgufProblem(_ptr(x), _ptr(p.codes), _ptr(p.scales), _ptr(y), p.n, p.k)
+    words = []
+    for x, p, y in zip(xs, ps, ys):
+        words += (x.data_ptr(), p.codes.data_ptr(), p.scales.data_ptr(), y.data_ptr(), p.n, p.k)
+    arr = _problem_array(ffi.GgufProblem, words)
     ffi.call("castforge_hip_gemv_gguf_q4_0_planes_batched", arr, len(ps), m, yd, _stream(xs[0]))
 
 
