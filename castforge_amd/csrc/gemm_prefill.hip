@@ -553,7 +553,7 @@ void prefill_i4_kernel(PfArgs a) {
     constexpr int kDma = kRowsX / 4;         // 1 KB buffer -> LDS loads per wave and block
     constexpr int kLoads = kDma + I * (kQ8 ? 9 : kQ4 ? 3 : kSG ? 6 : 4);  // vector-memory loads per wave and block
     static_assert(!kI8 || I * 4 == kLoads - kDma, "INT8: 4 code loads per row block");
-    static_assert(I >= 1 && kRowsX % 16 == 0 && S * kStage <= 160 * 1024, "tile / LDS budget");
+    static_assert(I >= 1 && kRowsX % 4 == 0 && S * kStage <= 160 * 1024, "tile / LDS budget");
     extern __shared__ __align__(16) uint8_t lds[];
 
     const int M = a.M, N = a.N, K = a.K;
@@ -594,12 +594,12 @@ void prefill_i4_kernel(PfArgs a) {
         vs[i] = row * static_cast<uint32_t>(GP) * 2u;
         vz[i] = row * static_cast<uint32_t>(ZW) * 4u;
     }
-    // lane offsets of the x loads: load t writes rows 4 t .. 4 t + 3 of the wave's BM / 4;
+    // lane offsets of the x loads: load t writes rows 4 t .. 4 t + 3 of the wave's BM / NW;
     // lane -> row 4 t + lane / 16, physical chunk lane % 16 (logical chunk ^ (row & 15))
     uint32_t lv[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-        const int r = 4 * u + (lane >> 4);
+        const int r = kRowsX * wave + 4 * u + (lane >> 4);
         lv[u] = static_cast<uint32_t>((lane >> 4) * K * 2 + (((lane & 15) ^ (r & 15)) * 16));
     }
 
@@ -703,7 +703,7 @@ void prefill_i4_kernel(PfArgs a) {
         const float q3 = __builtin_fmaf(static_cast<float>(p3.x), kOne, co), q7 = __builtin_fmaf(static_cast<float>(p3.y), kOne, co);
         return __builtin_bit_cast(bf16x8_t, make_uint4(pack_hi16(q0, q1), pack_hi16(q2, q3), pack_hi16(q4, q5), pack_hi16(q6, q7)));
     };
-    // Q8_0: 8 signed codes (two words, k order) -> 4 bf16 pairs of exact q: (w & 0x00FF00FF) ^
+    // INT8: 8 signed codes (two words, k order) -> 4 bf16 pairs of exact q: (w & 0x00FF00FF) ^
     // 0x64806480 is the f16 pair 1024 + (q + 128), and v_fma_mix_f32 subtracts 1152
     const uint32_t kM8 = opaque(0x00FF00FFu), kC8 = opaque(0x64806480u);
     auto decode8 = [&](uint32_t w0, uint32_t w1) __attribute__((always_inline)) {
@@ -716,6 +716,30 @@ void prefill_i4_kernel(PfArgs a) {
         const float q4 = __builtin_fmaf(static_cast<float>(b0.x), kOne, c), q6 = __builtin_fmaf(static_cast<float>(b0.y), kOne, c);
         const float q5 = __builtin_fmaf(static_cast<float>(b1.x), kOne, c), q7 = __builtin_fmaf(static_cast<float>(b1.y), kOne, c);
         return __builtin_bit_cast(bf16x8_t, make_uint4(pack_hi16(q0, q1), pack_hi16(q2, q3), pack_hi16(q4, q5), pack_hi16(q6, q7)));
+    };
+    // Q8_0: the same bits by one sign-extending byte conversion (SDWA) per code, 12 instructions against
+    // 18 (M = 4096, n = 11008, k = 4096: 555 us against 575; INT8, without folds, 398 against 389)
+    auto decode8b = [&](uint32_t w0, uint32_t w1) __attribute__((always_inline)) {
+        float q[8];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            q[j] = static_cast<float>(static_cast<int8_t>(w0 >> (8 * j)));
+            q[4 + j] = static_cast<float>(static_cast<int8_t>(w1 >> (8 * j)));
+        }
+        return __builtin_bit_cast(bf16x8_t, make_uint4(pack_hi16(q[0], q[1]), pack_hi16(q[2], q[3]), pack_hi16(q[4], q[5]), pack_hi16(q[6], q[7])));
+    };
+    // Q4_0: 8 codes -> 16 (q - 8) as bf16, exact: a nibble in the high half of a byte, its top bit
+    // flipped, is the signed byte 16 (q - 8); the 1/16 is in the block's d (15 instructions against 17;
+    // the same shape 479 us against 496)
+    auto decode4b = [&](uint32_t w) __attribute__((always_inline)) {
+        const uint32_t e = ((w << 4) & 0xF0F0F0F0u) ^ 0x80808080u, o = (w & 0xF0F0F0F0u) ^ 0x80808080u;
+        float q[8];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            q[2 * j] = static_cast<float>(static_cast<int8_t>(e >> (8 * j)));
+            q[2 * j + 1] = static_cast<float>(static_cast<int8_t>(o >> (8 * j)));
+        }
+        return __builtin_bit_cast(bf16x8_t, make_uint4(pack_hi16(q[0], q[1]), pack_hi16(q[2], q[3]), pack_hi16(q[4], q[5]), pack_hi16(q[6], q[7])));
     };
 
     // One set of partials.  Block b's first MFMA step overwrites pair (i, j) only right after
@@ -802,11 +826,12 @@ void prefill_i4_kernel(PfArgs a) {
                 if constexpr (kQ8 || kI8) {
                     // Q8_0: block kk / 2, piece 2 h + (kk & 1); INT8: words 2 kk, 2 kk + 1
                     const uint4 q = r.w[i][kk >> 1];
-                    wf[i] = (kk & 1) ? decode8(q.z, q.w) : decode8(q.x, q.y);
+                    const uint32_t w0 = (kk & 1) ? q.z : q.x, w1 = (kk & 1) ? q.w : q.y;
+                    wf[i] = kI8 ? decode8(w0, w1) : decode8b(w0, w1);
                 } else {
                     const uint4 q = r.w[i][half];
                     const uint32_t word = comp == 0 ? q.x : comp == 1 ? q.y : comp == 2 ? q.z : q.w;
-                    wf[i] = decode(word, ce[i], co[i]);
+                    wf[i] = FMT == FMT_Q4G ? decode4b(word) : decode(word, ce[i], co[i]);
                 }
             }
             // Q4_0: a new 32-wide block (and scale) every two steps
@@ -841,7 +866,7 @@ void prefill_i4_kernel(PfArgs a) {
 #pragma unroll
                 for (int i = 0; i < I; ++i) {
                     const uint32_t dw = r.s[i][kk >> 2];
-                    sc_prev[i] = f16_to_f32(static_cast<uint16_t>((kk & 2) ? (dw >> 16) : (dw & 0xFFFFu)));
+                    sc_prev[i] = f16_to_f32(static_cast<uint16_t>((kk & 2) ? (dw >> 16) : (dw & 0xFFFFu))) * (kQ8 ? 1.0f : 0.0625f);
                 }
             }
         });
@@ -1026,18 +1051,22 @@ void launch_fmt(const PfArgs &a, hipStream_t st) {
 // 290; 4096 x 11008 (16 n-tiles) at M = 256 / 512: 143 / 143 us against 121 / 199.
 // CASTFORGE_PREFILL_I4=0 keeps every INT4 problem on the generic kernel, =1 sends every one
 // whose groups allow it to the one-MFMA kernel.
-bool i4_eligible(const PfArgs &a, int fmt) {
+// Where qsplit_kernel takes a problem too, it has already left it to this kernel by its cost, and the
+// thresholds (against the generic kernel) do not apply (INT8 11008 x 4096 at M = 384, 129 tiles: 55 us
+// against 71 on the generic kernel).
+bool i4_eligible(const PfArgs &a, int fmt, bool split_ok) {
     if (fmt == FMT_I4G32 || fmt == FMT_I4G64) {
         if (a.K % kI4KB != 0) return false;
     } else if (fmt == FMT_Q4G || fmt == FMT_Q8G || fmt == FMT_INT8 ? a.K % kI4KB != 0
                                                                     : (a.group % kI4KB != 0 || a.K % a.group != 0)) {
         return false;
     }
-    if (static_cast<int64_t>(128) * a.K * 2 >= (int64_t{1} << 31)) return false;
+    if (static_cast<int64_t>(256) * a.K * 2 >= (int64_t{1} << 31)) return false;
     if (const char *e = std::getenv("CASTFORGE_PREFILL_I4")) {
         if (std::strcmp(e, "0") == 0) return false;
         if (std::strcmp(e, "1") == 0) return true;
     }
+    if (split_ok) return true;
     const int64_t cus = cu_count();
     const int64_t tiles = ((a.M + 127) / 128) * static_cast<int64_t>((a.N + kI4BN - 1) / kI4BN);
     // INT4: one tile per 6 CUs.  The GGUF forms fold every two MFMA steps and INT8's generic
@@ -1050,7 +1079,32 @@ bool i4_eligible(const PfArgs &a, int fmt) {
     return 6 * tiles >= cus;
 }
 
+// Rows of x per one-MFMA tile, by rounds of tiles over the CUs: 128; 96 for the formats whose tile
+// then takes 0.85 of the time (us a round at k = 4096, 128 / 96: INT4 65 / 54, Q4_0 76 / 65, Q8_0 90 /
+// 78; INT8, with no folds to save, 50 / 55), so a nearly empty last round is shed (Q8_0, n = 11008 at
+// M = 1500, 516 tiles: 264 -> 237 us); 256 for INT8 where half the decodes outweigh the coarser
+// rounds (M = 4096: 389 -> 369 us; 1.9 times the time a round).
+enum PfRows { PF_ROWS_96, PF_ROWS_128, PF_ROWS_256 };
+int64_t pf_rounds(int64_t m, int64_t n, int64_t bm) {
+    const int64_t cus = cu_count();
+    return ((m + bm - 1) / bm * ((n + kI4BN - 1) / kI4BN) + cus - 1) / cus;
+}
+PfRows prefill_rows(int fmt, int64_t m, int64_t n) {
+    const double r128 = static_cast<double>(pf_rounds(m, n, 128));
+    if (fmt == FMT_INT8) return 1.9 * static_cast<double>(pf_rounds(m, n, 256)) < r128 ? PF_ROWS_256 : PF_ROWS_128;
+    return 0.85 * static_cast<double>(pf_rounds(m, n, 96)) < r128 ? PF_ROWS_96 : PF_ROWS_128;
+}
+
 }  // namespace
+
+// Rounds of 128-row tiles that the one-MFMA kernel's tiles take the time of (INT4 groups of 32 / 64
+// and INT8 at 128 rows: the tile heights of prefill_rows differ little there).
+double prefill_cost(int fmt, bool rows96, int64_t m, int64_t n) {
+    const double r128 = static_cast<double>(pf_rounds(m, n, 128));
+    return rows96 && prefill_rows(fmt, m, n) == PF_ROWS_96 ? 0.85 * static_cast<double>(pf_rounds(m, n, 96)) : r128;
+}
+
+bool qsplit_ok(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes, const void *scales);
 
 // Routes one problem to the prefill MFMA kernel when its shape allows it.
 bool prefill_try(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group,
@@ -1064,14 +1118,25 @@ bool prefill_try(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, in
     if (!aligned(x, 16) || !aligned(codes, 16)) return false;
     PfArgs a{x, codes, scales, zeros, y, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k),
              static_cast<int>(fmt == FMT_INT8 ? BK : group), per_row, y_bf16, (n % 4 == 0 && aligned(y, 16)) ? 1 : 0, 0, 0};
-    if (fmt == FMT_INT4 && i4_eligible(a, fmt)) launch_i4<128, CFH_PF_I4_DEPTH, CFH_PF_I4_WAVES, FMT_INT4>(a, st);
-    else if (fmt == FMT_INT4 && a.group == 32 && i4_eligible(a, FMT_I4G32))
+    const PfRows rows = prefill_rows(fmt, m, n);
+    const bool split_ok = qsplit_ok(fmt, x, m, n, k, group, codes, scales);
+    if (fmt == FMT_INT4 && i4_eligible(a, fmt, split_ok)) {
+        if (rows == PF_ROWS_96) launch_i4<96, CFH_PF_I4_DEPTH, CFH_PF_I4_WAVES, FMT_INT4>(a, st);
+        else launch_i4<128, CFH_PF_I4_DEPTH, CFH_PF_I4_WAVES, FMT_INT4>(a, st);
+    } else if (fmt == FMT_INT4 && a.group == 32 && i4_eligible(a, FMT_I4G32, split_ok)) {
         launch_i4<128, CFH_PF_Q4_DEPTH, CFH_PF_I4_WAVES, FMT_I4G32, 1>(a, st);  // two W sets: three spill
-    else if (fmt == FMT_INT4 && a.group == 64 && i4_eligible(a, FMT_I4G64))
+    } else if (fmt == FMT_INT4 && a.group == 64 && i4_eligible(a, FMT_I4G64, split_ok)) {
         launch_i4<128, CFH_PF_Q4_DEPTH, CFH_PF_I4_WAVES, FMT_I4G64>(a, st);
-    else if (fmt == FMT_INT8 && i4_eligible(a, fmt)) launch_i4<128, CFH_PF_Q8_DEPTH, CFH_PF_I4_WAVES, FMT_INT8, CFH_PF_Q8_WDEPTH>(a, st);
-    else if (fmt == FMT_Q4G && i4_eligible(a, fmt)) launch_i4<128, CFH_PF_Q4_DEPTH, CFH_PF_I4_WAVES, FMT_Q4G>(a, st);
-    else if (fmt == FMT_Q8G && i4_eligible(a, fmt)) launch_i4<128, CFH_PF_Q8_DEPTH, CFH_PF_I4_WAVES, FMT_Q8G, CFH_PF_Q8_WDEPTH>(a, st);
+    } else if (fmt == FMT_INT8 && i4_eligible(a, fmt, split_ok)) {
+        if (rows == PF_ROWS_256) launch_i4<256, 1, CFH_PF_I4_WAVES, FMT_INT8, 1>(a, st);
+        else launch_i4<128, CFH_PF_Q8_DEPTH, CFH_PF_I4_WAVES, FMT_INT8, CFH_PF_Q8_WDEPTH>(a, st);
+    } else if (fmt == FMT_Q4G && i4_eligible(a, fmt, split_ok)) {
+        if (rows == PF_ROWS_96) launch_i4<96, CFH_PF_Q4_DEPTH, CFH_PF_I4_WAVES, FMT_Q4G>(a, st);
+        else launch_i4<128, CFH_PF_Q4_DEPTH, CFH_PF_I4_WAVES, FMT_Q4G>(a, st);
+    } else if (fmt == FMT_Q8G && i4_eligible(a, fmt, split_ok)) {
+        if (rows == PF_ROWS_96) launch_i4<96, CFH_PF_Q8_DEPTH, CFH_PF_I4_WAVES, FMT_Q8G, CFH_PF_Q8_WDEPTH>(a, st);
+        else launch_i4<128, CFH_PF_Q8_DEPTH, CFH_PF_I4_WAVES, FMT_Q8G, CFH_PF_Q8_WDEPTH>(a, st);
+    }
     else if (fmt == FMT_INT4) launch_fmt<FMT_INT4>(a, st);
     else if (fmt == FMT_NF4) launch_fmt<FMT_NF4>(a, st);
     else if (fmt == FMT_Q4G) launch_fmt<FMT_Q4G>(a, st);

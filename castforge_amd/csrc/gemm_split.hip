@@ -25,6 +25,10 @@
 #include "cfh_common.hpp"
 
 namespace cfh {
+
+// what the one-MFMA prefill kernel takes for M x N, in rounds of 128-row tiles (gemm_prefill.hip)
+double prefill_cost(int fmt, bool rows96, int64_t m, int64_t n);
+
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -495,9 +499,9 @@ void launch(QsArgs a, hipStream_t st) {
 // (12 / 12 / 14); then 64 x 64 (18 / 18 / 23 a round) or, above M = 64, 64 (n) x 128 (35 / 28 / 40)
 // where its rounds cost less.  Every shape up to M = 64 sums the same chunks in the same order, so a
 // batch gives the bits of one call per problem.
-// False (M > 64) where the one-MFMA prefill kernel's 256 (n) x 128 tiles cost less still: a round of
-// it takes rpf rounds of 64 x 64 however few its tiles (INT4, 4096 x 4096 at M = 512: 34 us here
-// against 59; 11008 x 4096 at M = 512: 92 against 68).
+// False (M > 64) where the one-MFMA prefill kernel costs less still: a round of its 256 (n) x 128
+// tiles takes rpf rounds of 64 x 64 however few its tiles (INT4, 4096 x 4096 at M = 512: 33 us here
+// against 59; 11008 x 4096 at M = 512: 92 against 68; 4096 x 11008 at M = 603: 104 against 123).
 template <int FMT, int FMT_SMALL>
 bool launch_fmt(const QsArgs &a, double r128, double rpf, hipStream_t st) {
     const int64_t cus = cu_count();
@@ -522,7 +526,7 @@ bool launch_fmt(const QsArgs &a, double r128, double rpf, hipStream_t st) {
         return true;
     }
     const double c64 = rounds(tiles(64, 64)), c128 = r128 * rounds(tiles(64, 128));
-    if (std::min(c64, c128) > rpf * rounds(tiles(256, 128))) return false;
+    if (std::min(c64, c128) > rpf * prefill_cost(FMT, FMT != FMT_INT8 && a.p[0].group != 64 && FMT != FMT_I4G32, a.M, a.p[0].N)) return false;
     if (c64 <= c128) launch<FMT, 2, 2, 8, 2>(a, st);
     else launch<FMT, 2, 4, 4, 2>(a, st);
     return true;
@@ -530,10 +534,10 @@ bool launch_fmt(const QsArgs &a, double r128, double rpf, hipStream_t st) {
 
 bool launch_any(int fmt, const QsArgs &a, hipStream_t st) {
     if (fmt == FMT_INT8) return launch_fmt<FMT_INT8, FMT_I8S>(a, 1.5, 3.1, st);
-    if (fmt == FMT_Q4G) return launch_fmt<FMT_Q4G, FMT_Q4G>(a, 1.75, 3.5, st);
-    if (fmt == FMT_Q8G) return launch_fmt<FMT_Q8G, FMT_Q8G>(a, 1.75, 4.1, st);
+    if (fmt == FMT_Q4G) return launch_fmt<FMT_Q4G, FMT_Q4G>(a, 1.75, 4.0, st);
+    if (fmt == FMT_Q8G) return launch_fmt<FMT_Q8G, FMT_Q8G>(a, 1.75, 4.6, st);
     if (a.p[0].group == 32) return launch_fmt<FMT_I4G32, FMT_I4G32>(a, 1.65, 3.5, st);
-    return launch_fmt<FMT_INT4, FMT_INT4>(a, 1.95, 3.5, st);
+    return launch_fmt<FMT_INT4, FMT_INT4>(a, 1.95, 4.0, st);
 }
 
 QsProb prob(const uint16_t *x, int64_t n, int64_t k, int64_t group, const void *codes, const void *scales,

@@ -53,3 +53,20 @@ def test_split_vs_float64(cuda, fmt, k, m, n):
         yy = torch.empty_like(y)
         run_batched(x, yy)
         assert torch.equal(yy, y)
+
+
+# (m, n): one round of 96-row tiles against one or two of 128; two rounds of 128-row tiles against one
+# of 256 (INT8)
+@pytest.mark.parametrize("fmt", ["int4_128", "int8_channel", "q4_0", "q8_0"])
+@pytest.mark.parametrize("m,n", [(97, 300), (1536, 5376), (1601, 5377)])
+def test_prefill_tile_heights_vs_float64(cuda, fmt, m, n, monkeypatch):
+    """The one-MFMA prefill kernel at each of its tile heights (96, 128, 256 rows by rounds over the
+    CUs), row and column remainders included."""
+    monkeypatch.setenv("CASTFORGE_PREFILL_I4", "1")
+    k = 256
+    wd, run, _ = _weight(fmt, n, k, cuda)
+    x = torch.from_numpy(synth.activations_bf16(35, m, m, k).view(np.int16)).view(torch.bfloat16).to(cuda)
+    ref, mag = x.double() @ wd.double().t(), x.double().abs() @ wd.double().abs().t()
+    bound = (k / 16 + k / 32 + 10) * 2.0 ** -24 * mag
+    y = run(x, torch.float32)
+    assert bool(((y.double() - ref).abs() <= bound).all()), (fmt, m, n)
