@@ -82,11 +82,13 @@ def test_fp8_gemm_vs_oracle(cuda, m, n, k, exact):
 
 
 # K split over waves: one half chunk (k = 64), an odd number of 64-wide halves, fewer chunks than
-# waves, many chunks; tile remainders in m and n.  The last three have more than two 32 x 32 tiles
-# per CU (64 x 64 tiles), the very last more than six 64 x 64 (256 x 256 tiles).
+# waves, many chunks; tile remainders in m and n.  From 520 x 1050 on there are more than two
+# 32 x 32 tiles per CU: 64 x 64, 128 x 128 (the third of them), and, by rounds over 256 CUs, 256 x 128,
+# 256 x 192 and 256 x 256 tiles.
 @pytest.mark.parametrize("exact", [True, False])
 @pytest.mark.parametrize("m,n,k", [(1, 1, 64), (31, 33, 192), (32, 32, 512), (33, 65, 576), (2, 200, 4160),
-                                   (520, 1050, 192), (545, 1024, 1088), (2500, 2900, 64)])
+                                   (520, 1050, 192), (545, 1024, 1088), (1000, 4001, 64), (2047, 4090, 64),
+                                   (2999, 4001, 64), (4001, 4000, 64), (4095, 4090, 128)])
 def test_fp8_gemm_split_edges(cuda, m, n, k, exact):
     a = synth.fp8_inputs(85, m, m, k)
     w = synth.fp8_inputs(85, n, n, k) * np.float32(0.02)
