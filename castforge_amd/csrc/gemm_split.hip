@@ -1,6 +1,6 @@
-// Quantized-weight products of small and mid-sized M on one bf16 MFMA per product, K split over
-// the waves of a workgroup: y[m, n] = sum_k x[m, k] W[n, k] for INT4 (groups of 32, 64 or a
-// multiple of 128), INT8 and the GGUF Q4_0 / Q8_0 planes.
+// Quantized-weight products of small and mid-sized M on one bf16 MFMA per product (NF4: two), K
+// split over the waves of a workgroup: y[m, n] = sum_k x[m, k] W[n, k] for INT4 (groups of 32, 64 or
+// a multiple of 64), INT8, NF4 (M > 16) and the GGUF Q4_0 / Q8_0 planes.
 //
 // The weight operand is the exact integer (q - z, q or q - 8) as bf16 and x is the bf16 it is, as
 // in prefill_i4_kernel; each 64-wide chunk (32-wide where the format scales every 32) sums into a
@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
+#include <cstring>
 
 #include "../../include/castforge_hip.h"
 #include "cfh_common.hpp"
@@ -36,18 +37,19 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
 // numbers as in gemm_prefill.hip; FMT_I8S: INT8 with a partial per chunk (any finite x)
-enum Fmt { FMT_INT4 = 0, FMT_INT8 = 1, FMT_Q4G = 3, FMT_Q8G = 4, FMT_I4G32 = 5, FMT_I8S = 7 };
+enum Fmt { FMT_INT4 = 0, FMT_INT8 = 1, FMT_NF4 = 2, FMT_Q4G = 3, FMT_Q8G = 4, FMT_I4G32 = 5, FMT_I8S = 7 };
 template <int FMT> constexpr bool kBytes = FMT == FMT_INT8 || FMT == FMT_I8S || FMT == FMT_Q8G;  // 8-bit codes
 template <int FMT> constexpr bool kRowScale = FMT == FMT_INT8 || FMT == FMT_I8S;                 // one f32 scale per row
 
 // The weight operand is the integer times 2^-kShift, undone in the scale: a partial of 64 (32)
 // products then stays below the largest |x|, so it is finite for every finite x, and the smallest
 // products (bf16 subnormal x) still have their last bit at or above 2^-149.
-template <int FMT> constexpr int kShift = FMT == FMT_INT8 ? 0 : FMT == FMT_I8S ? 14 : FMT == FMT_Q8G ? 13 : 11;
+template <int FMT> constexpr int kShift = FMT == FMT_INT8 || FMT == FMT_NF4 ? 0 : FMT == FMT_I8S ? 14 : FMT == FMT_Q8G ? 13 : 11;
 
 constexpr int kXcds = 8;
 constexpr int kChunk = 64;          // K elements of a chunk
 constexpr int kXRow = kChunk * 2;   // bytes of x per row and chunk
+constexpr int kCopies = 16;         // of the NF4 decode table
 
 struct QsProb {
     const uint16_t *x;
@@ -89,7 +91,7 @@ __device__ __forceinline__ int xswz(int r, int c) { return c ^ ((r >> 1) & 7); }
 
 template <int FMT> constexpr bool fold32() { return FMT == FMT_Q4G || FMT == FMT_Q8G || FMT == FMT_I4G32; }
 // vector-memory loads of one chunk per 32 weight rows: codes, scales, zero points
-template <int FMT> constexpr int w_loads() { return kRowScale<FMT> ? 2 : FMT == FMT_INT4 ? 1 : FMT == FMT_I4G32 ? 4 : 3; }
+template <int FMT> constexpr int w_loads() { return kRowScale<FMT> || FMT == FMT_NF4 ? 2 : FMT == FMT_INT4 ? 1 : FMT == FMT_I4G32 ? 4 : 3; }
 
 // One lane's codes and scales of a chunk (its row of 32, its half h of the MFMA's K).
 template <int FMT>
@@ -113,7 +115,7 @@ struct WAddr {
 };
 
 template <int FMT>
-__device__ __forceinline__ void load_w(const WAddr &A, int i, int c, WSet<FMT> &r) {
+__device__ __forceinline__ void load_w(const WAddr &A, int i, int c, int cpg, WSet<FMT> &r) {
     const uint32_t vw = A.vw + i * A.row_w, vs = A.vs + i * A.row_s;
     if constexpr (kRowScale<FMT>) {
         // bytes 32 h .. 32 h + 31 of the row's 64
@@ -139,6 +141,9 @@ __device__ __forceinline__ void load_w(const WAddr &A, int i, int c, WSet<FMT> &
         r.w[0] = make_uint4(p.x, p.y, q.x, q.y);
         r.s = __builtin_amdgcn_raw_buffer_load_b32(A.rs, vs, c * 4, 0);
         r.z = __builtin_amdgcn_raw_buffer_load_b32(A.rz, A.vz + i * A.row_z, (c >> 2) * 4, 0);
+    } else if constexpr (FMT == FMT_NF4) {
+        r.w[0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(A.rw, vw, c * 32, 0));
+        r.s = __builtin_amdgcn_raw_buffer_load_b32(A.rs, vs, (c >> cpg) * 4, 0);  // cpg: log2 of chunks per block
     } else {
         r.w[0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(A.rw, vw, c * 32, 0));
     }
@@ -209,7 +214,7 @@ __device__ __forceinline__ void chunk_step(const uint8_t *__restrict__ cur, uint
     if (refill) {
         issue_x<J>(rx, nxt, lv, K, c_next);
 #pragma unroll
-        for (int i = 0; i < I; ++i) load_w<FMT>(A, i, c_next, wn[i]);
+        for (int i = 0; i < I; ++i) load_w<FMT>(A, i, c_next, cpg, wn[i]);
     }
     wait_vm_fence<(S - 1) * kLoads>();
     constexpr float kUp = static_cast<float>(1 << kShift<FMT>);
@@ -247,8 +252,20 @@ __device__ __forceinline__ void chunk_step(const uint8_t *__restrict__ cur, uint
         }
 #pragma unroll
         for (int i = 0; i < I; ++i) {
-            bf16x8_t wf;
-            if constexpr (FMT == FMT_INT8) {
+            bf16x8_t wf, wl;
+            if constexpr (FMT == FMT_NF4) {
+                // the table's row of a code byte holds, per copy, the T_hi pair and the T_lo pair
+                const uint4 q = w[i].w[0];
+                const uint32_t word = kk == 0 ? q.x : kk == 1 ? q.y : kk == 2 ? q.z : q.w;
+                uint32_t hi[4], lo[4];
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const uint2 e = *reinterpret_cast<const uint2 *>(sz + ((word >> (8 * b)) & 0xFFu) * (2 * kCopies) + 2 * (fr % kCopies));
+                    hi[b] = e.x, lo[b] = e.y;
+                }
+                wf = __builtin_bit_cast(bf16x8_t, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+                wl = __builtin_bit_cast(bf16x8_t, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+            } else if constexpr (FMT == FMT_INT8) {
                 const uint4 q = w[i].w[kk >> 1];
                 wf = (kk & 1) ? decode8(q.z, q.w) : decode8(q.x, q.y);
             } else if constexpr (FMT == FMT_I8S) {
@@ -273,11 +290,13 @@ __device__ __forceinline__ void chunk_step(const uint8_t *__restrict__ cur, uint
                 } else {
                     part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[j], wf, part[i][j], 0, 0, 0);
                 }
+                if constexpr (FMT == FMT_NF4) part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[j], wl, part[i][j], 0, 0, 0);
             }
         }
         if constexpr (FMT != FMT_INT8 && (fold32<FMT>() ? (kk & 1) == 1 : kk == 3)) {
 #pragma unroll
             for (int i = 0; i < I; ++i) {
+                if constexpr (FMT == FMT_NF4) sc[i] = __uint_as_float(w[i].s);
                 if constexpr (fold32<FMT>()) sc[i] = f16_to_f32(static_cast<uint16_t>(kk == 1 ? (w[i].s & 0xFFFFu) : (w[i].s >> 16))) * kUp;
 #pragma unroll
                 for (int j = 0; j < J; ++j)
@@ -292,11 +311,20 @@ __device__ __forceinline__ void chunk_step(const uint8_t *__restrict__ cur, uint
     });
 }
 
-// LDS of a workgroup: the x rings and (INT4) the tile's `groups` scales and zero points, later the
-// waves' partial tiles.
+// The NF4 table of QLoRA, as the evaluator's f32 values.  In LDS: for each code byte (two codes),
+// kCopies copies of its T_hi = RNE(T) and T_lo = RNE(T - T_hi) bf16 pairs, the operand words of two MFMAs
+// (16 copies: 32 KB, lanes r and r + 16 share one, so a read takes at most two passes).
+__constant__ float kNf4S[16] = {
+    -1.0f, -0.6961928009986877f, -0.5250730514526367f, -0.39491748809814453f,
+    -0.28444138169288635f, -0.18477343022823334f, -0.09105003625154495f, 0.0f,
+    0.07958029955625534f, 0.16093020141124725f, 0.24611230194568634f, 0.33791524171829224f,
+    0.44070982933044434f, 0.5626170039176941f, 0.7229568362236023f, 1.0f};
+
+// LDS of a workgroup: the x rings and the tile's `groups` scales and zero points (INT4) or the decode
+// table (NF4), later the waves' partial tiles.
 template <int FMT, int I, int J, int NW, int S>
 constexpr int64_t lds_bytes(int64_t groups) {
-    const int64_t ring = NW * S * 32 * J * kXRow + (FMT == FMT_INT4 ? groups * 32 * I * 4 : 0), sums = NW * 32 * J * (32 * I + 4) * 4;
+    const int64_t ring = NW * S * 32 * J * kXRow + (FMT == FMT_INT4 ? groups * 32 * I * 4 : FMT == FMT_NF4 ? 256 * kCopies * 8 : 0), sums = NW * 32 * J * (32 * I + 4) * 4;
     return ring > sums ? ring : sums;
 }
 constexpr int64_t kLdsMax = 160 * 1024;
@@ -330,20 +358,24 @@ __global__ __launch_bounds__(64 * NW) void qsplit_kernel(QsArgs g) {
     WAddr A;
     const int row_bytes = kBytes<FMT> ? K : K / 2;
     // scales per row: GGUF planes 8 ceil(K / 32 / 8), INT4 8 ceil(G / 8)
+    // (NF4: f32 absmax, K / block)
     const int G = FMT == FMT_INT4 || FMT == FMT_I4G32 ? K / a.group : K / 32;
     const int ZW = (G + 7) / 8, GP = ZW * 8;
     const uint32_t nv = static_cast<uint32_t>(min(kBN, N - n0));
     A.rw = make_rsrc(static_cast<const uint8_t *>(a.codes) + static_cast<int64_t>(n0) * row_bytes, nv * row_bytes);
-    A.rs = make_rsrc(static_cast<const uint16_t *>(a.scales) + static_cast<int64_t>(n0) * (kRowScale<FMT> ? 0 : GP), kRowScale<FMT> ? 0 : nv * GP * 2);
+    const int NB = FMT == FMT_NF4 ? K / a.group : 0;  // absmax blocks per row
+    A.rs = FMT == FMT_NF4 ? make_rsrc(static_cast<const float *>(a.scales) + static_cast<int64_t>(n0) * NB, nv * NB * 4)
+                          : make_rsrc(static_cast<const uint16_t *>(a.scales) + static_cast<int64_t>(n0) * (kRowScale<FMT> ? 0 : GP),
+                                      kRowScale<FMT> ? 0 : nv * GP * 2);
     constexpr bool kZeros = FMT == FMT_INT4 || FMT == FMT_I4G32;
     A.rz = make_rsrc(a.zeros + static_cast<int64_t>(n0) * (kZeros ? ZW : 0), kZeros ? nv * ZW * 4 : 0);
-    A.vw = fr * row_bytes + (FMT == FMT_INT4 ? 16 : FMT == FMT_I4G32 ? 8 : 32) * h;
-    A.vs = fr * GP * 2;
+    A.vw = fr * row_bytes + (FMT == FMT_INT4 || FMT == FMT_NF4 ? 16 : FMT == FMT_I4G32 ? 8 : 32) * h;
+    A.vs = FMT == FMT_NF4 ? fr * NB * 4 : fr * GP * 2;
     A.vz = fr * ZW * 4;
     A.row_w = 32 * row_bytes;
-    A.row_s = 32 * GP * 2;
+    A.row_s = FMT == FMT_NF4 ? 32 * NB * 4 : 32 * GP * 2;
     A.row_z = 32 * ZW * 4;
-    const int cpg = FMT == FMT_INT4 ? a.group / kChunk : 1;
+    const int cpg = FMT == FMT_INT4 ? a.group / kChunk : FMT == FMT_NF4 ? __builtin_ctz(static_cast<uint32_t>(a.group / kChunk)) : 1;
 
     auto opaque = [](uint32_t v) __attribute__((always_inline)) {
         asm("" : "+v"(v));
@@ -384,7 +416,7 @@ __global__ __launch_bounds__(64 * NW) void qsplit_kernel(QsArgs g) {
             asm volatile("" ::: "memory");  // the waits count whole chunks
             issue_x<J>(rx, ring + t * kStage, lv, K, c_of(t));
 #pragma unroll
-            for (int i = 0; i < I; ++i) load_w<FMT>(A, i, c_of(t), ws[t][i]);
+            for (int i = 0; i < I; ++i) load_w<FMT>(A, i, c_of(t), cpg, ws[t][i]);
         }
     });
     // INT4: every group's scale (f16, low half) and zero point of the tile's rows, [group][row], once
@@ -400,6 +432,16 @@ __global__ __launch_bounds__(64 * NW) void qsplit_kernel(QsArgs g) {
 #pragma unroll
             for (int q = 0; q < 8; ++q)
                 if (8 * g8 + q < G) sz[(8 * g8 + q) * kBN + r] = ((dw[q >> 1] >> (16 * (q & 1))) & 0xFFFFu) | ((z >> (4 * q)) & 15u) << 16;
+        }
+        __syncthreads();
+    }
+    if constexpr (FMT == FMT_NF4) {
+        for (int o = threadIdx.x; o < 256 * kCopies; o += 64 * NW) {
+            const int v = o / kCopies;
+            const float t0 = kNf4S[v & 15], t1 = kNf4S[v >> 4];
+            const uint32_t hi = f32x2_to_bf16x2_rne(t0, t1);
+            const uint32_t lo = f32x2_to_bf16x2_rne(t0 - __uint_as_float(hi << 16), t1 - __uint_as_float(hi & 0xFFFF0000u));
+            *reinterpret_cast<uint2 *>(sz + 2 * o) = make_uint2(hi, lo);
         }
         __syncthreads();
     }
@@ -532,8 +574,30 @@ bool launch_fmt(const QsArgs &a, double r128, double rpf, hipStream_t st) {
     return true;
 }
 
+// NF4 (two MFMAs per product), us per round of 256 workgroups at K = 4096: 32 x 32 tiles up to one per CU
+// (10), 64 (n) x 32 beyond for M <= 32 (16), 32 (n) x 64 up to one per CU (14), then 64 x 64 (23 a round),
+// which holds to the largest M (4096 x 4096 at M = 512 / 4096: 49 / 322 us; the kernel of 128 (n) x 64 tiles
+// over two or four K parts that served M > 16 before took 36 at M = 64, 49 and 326, and 997 against 766
+// for 4096 x 11008 at M = 4096).  All sum the same chunks in the same order.
+void launch_nf4(const QsArgs &a, hipStream_t st) {
+    const int64_t cus = cu_count();
+    const auto tiles = [&](int64_t bn, int64_t bm) {
+        int64_t t = 0;
+        for (int i = 0; i < a.count; ++i) t += (a.M + bm - 1) / bm * ((a.p[i].N + bn - 1) / bn);
+        return t;
+    };
+    if (tiles(32, 32) <= cus) launch<FMT_NF4, 1, 1, 8, 2>(a, st);
+    else if (a.M <= 32) launch<FMT_NF4, 2, 1, 8, 2>(a, st);
+    else if (tiles(32, 64) <= cus) launch<FMT_NF4, 1, 2, 8, 2>(a, st);
+    else launch<FMT_NF4, 2, 2, 8, 2>(a, st);
+}
+
 bool launch_any(int fmt, const QsArgs &a, hipStream_t st) {
     if (fmt == FMT_INT8) return launch_fmt<FMT_INT8, FMT_I8S>(a, 1.5, 3.1, st);
+    if (fmt == FMT_NF4) {
+        launch_nf4(a, st);
+        return true;
+    }
     if (fmt == FMT_Q4G) return launch_fmt<FMT_Q4G, FMT_Q4G>(a, 1.75, 4.0, st);
     if (fmt == FMT_Q8G) return launch_fmt<FMT_Q8G, FMT_Q8G>(a, 1.75, 4.6, st);
     if (a.p[0].group == 32) return launch_fmt<FMT_I4G32, FMT_I4G32>(a, 1.65, 3.5, st);
@@ -551,12 +615,19 @@ QsProb prob(const uint16_t *x, int64_t n, int64_t k, int64_t group, const void *
 // Whether qsplit_kernel takes a problem of M = m >= 2 rows.  The variables that choose a prefill
 // kernel keep M > 16 off it.
 bool qsplit_ok(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes, const void *scales) {
-    if (fmt != FMT_INT4 && fmt != FMT_INT8 && fmt != FMT_Q4G && fmt != FMT_Q8G) return false;
+    if (fmt != FMT_INT4 && fmt != FMT_INT8 && fmt != FMT_NF4 && fmt != FMT_Q4G && fmt != FMT_Q8G) return false;
+    // NF4: M > 16 (a partial reaches 64 |x|; up to 16 rows the skinny kernels take any finite x), blocks a
+    // power of two; CASTFORGE_NF4_MFMA=0 keeps it on the skinny / prefill kernels (for comparison)
+    if (fmt == FMT_NF4) {
+        if (m < 17 || k < 256 || group < kChunk || (group & (group - 1)) != 0 || k % group != 0) return false;
+        const char *e = std::getenv("CASTFORGE_NF4_MFMA");
+        if (e && std::strcmp(e, "0") == 0) return false;
+    }
     if (m < 2 || n < 1 || k < kChunk || k % kChunk != 0) return false;
     if (m > 0x7fffffff || n > 0x7fffffff) return false;
     // 32-bit buffer offsets over one tile's rows of x (128) and of codes (64)
     if (int64_t{128} * k * 2 >= (int64_t{1} << 31)) return false;
-    if (!aligned(x, 16) || !aligned(codes, 16) || !aligned(scales, fmt == FMT_INT8 ? 4 : 16)) return false;
+    if (!aligned(x, 16) || !aligned(codes, 16) || !aligned(scales, fmt == FMT_INT8 || fmt == FMT_NF4 ? 4 : 16)) return false;
     if (fmt == FMT_Q4G && (group != 32 || k % 128 != 0)) return false;
     if (fmt == FMT_Q8G && group != 32) return false;
     if (fmt == FMT_INT4) {
@@ -564,7 +635,7 @@ bool qsplit_ok(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int6
         // groups of 64 and more: the largest tile's scales and zero points next to the x rings
         if (group != 32 && lds_bytes<FMT_INT4, 2, 2, 8, 2>(k / group) > kLdsMax) return false;
     }
-    if (m > 16 && (std::getenv("CASTFORGE_PREFILL_I4") || std::getenv("CASTFORGE_PREFILL_TILE"))) return false;
+    if (fmt != FMT_NF4 && m > 16 && (std::getenv("CASTFORGE_PREFILL_I4") || std::getenv("CASTFORGE_PREFILL_TILE"))) return false;
     return true;
 }
 
@@ -578,7 +649,7 @@ bool qsplit_try(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int
     return launch_any(fmt, a, st);
 }
 
-// One launch over up to CFH_MAX_BATCH INT8 / INT4 / GGUF problems of one format and group (INT4:
+// One launch over up to CFH_MAX_BATCH INT8 / INT4 / NF4 / GGUF problems of one format and group (INT4:
 // whole multiples of 64) with the same M (2..64), each checked by qsplit_ok.
 void qsplit_batch(int fmt, int64_t m, int count, const uint16_t *const *x, const int64_t *n, const int64_t *k,
                   const int64_t *group, const void *const *codes, const void *const *scales, const uint32_t *const *zeros,

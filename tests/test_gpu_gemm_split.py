@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 # (m, n): 32 x 32 tiles (M <= 32; few tiles); 32 (n) x 64 (M <= 64, M > 64); 64 x 64 (M <= 64,
 # M > 64); 64 (n) x 128; one row and column past or short of a tile
-SHAPES = [(2, 1), (31, 65), (33, 64), (64, 97), (40, 4200), (70, 2803), (40, 9000), (130, 4000), (300, 3301)]
+SHAPES = [(2, 1), (31, 65), (19, 9000), (33, 64), (64, 97), (40, 4200), (70, 2803), (40, 9000), (130, 4000), (300, 3301)]
 
 
 def _weight(fmt, n, k, cuda):
@@ -23,6 +23,9 @@ def _weight(fmt, n, k, cuda):
         q, s = ops.quantize_int8(w, 8, gran)
         return (ops.dequantize_int8(q, s, gran), lambda x, o: ops.gemm_w8a16(x, q, s, gran, o),
                 lambda x, y: ops.gemv_w8a16_batched([x], [(q, s)], [y], gran))
+    if fmt.startswith("nf4"):
+        p = ops.quantize_nf4(w, int(fmt[4:]))
+        return ops.dequantize_nf4(p), lambda x, o: ops.gemm_nf4(x, p, o), lambda x, y: ops.gemv_nf4_batched([x], [p], [y])
     ty, size = (ffi.GGML_Q4_0, 18) if fmt == "q4_0" else (ffi.GGML_Q8_0, 34)
     rng = np.random.default_rng(n + k)
     raw = rng.integers(0, 256, (n * k // 32, size), dtype=np.uint8)
@@ -34,7 +37,7 @@ def _weight(fmt, n, k, cuda):
 # k: fewer 64-wide chunks than the workgroup's eight waves, and 18 chunks (some waves one more)
 @pytest.mark.parametrize("fmt,k", [("int4_32", 192), ("int4_64", 192), ("int4_64", 1152), ("int4_128", 1152),
                                    ("int4_256", 1280), ("int8_channel", 192), ("int8_tensor", 1152),
-                                   ("q4_0", 1152), ("q8_0", 192), ("q8_0", 1152)])
+                                   ("q4_0", 1152), ("q8_0", 192), ("q8_0", 1152), ("nf4_64", 256), ("nf4_128", 1152)])
 @pytest.mark.parametrize("m,n", SHAPES)
 def test_split_vs_float64(cuda, fmt, k, m, n):
     wd, run, run_batched = _weight(fmt, n, k, cuda)
@@ -44,12 +47,14 @@ def test_split_vs_float64(cuda, fmt, k, m, n):
     # f32 roundings on a path of one product: an MFMA step every 16 of K, a scale every 32, the sum of
     # eight waves and the dequantized weight's own; each at most 2^-24 of the magnitudes summed
     bound = (k / 16 + k / 32 + 10) * 2.0 ** -24 * mag
+    if fmt.startswith("nf4"):  # two MFMAs a step; T_hi + T_lo is within 2^-17 of the table value
+        bound += (k / 16 * 2.0 ** -24 + 2.0 ** -17) * mag
     y = run(x, torch.float32)
     assert bool(((y.cpu().double() - ref).abs() <= bound).all()), (fmt, m, n, k)
     yb = run(x, torch.bfloat16)
     assert torch.equal(yb, y.to(torch.bfloat16))
     # (batched INT4 takes groups of 128; a single GGUF call of two rows runs the M = 1 kernel)
-    if m <= 64 and fmt in ("int4_128", "int8_channel", "int8_tensor") or 2 < m <= 64 and fmt[0] == "q":
+    if m <= 64 and (fmt in ("int4_128", "int8_channel", "int8_tensor") or fmt[0] == "n" or m > 2 and fmt[0] == "q"):
         yy = torch.empty_like(y)
         run_batched(x, yy)
         assert torch.equal(yy, y)
