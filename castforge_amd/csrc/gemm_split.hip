@@ -194,25 +194,27 @@ __device__ __forceinline__ bf16x8_t decode8(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(bf16x8_t, make_uint4(pack_hi16(v[0], v[1]), pack_hi16(v[2], v[3]), pack_hi16(v[4], v[5]), pack_hi16(v[6], v[7])));
 }
 
-template <int J>
+// XL: 1 KB loads of x per chunk (8 rows each), the size of a stage: 4 J, or fewer where M <= 8 XL
+template <int XL>
 __device__ __forceinline__ void issue_x(rsrc_t rx, uint8_t *__restrict__ dst, const int (&lv)[2], int K, int c) {
 #pragma unroll
-    for (int t = 0; t < 4 * J; ++t)
+    for (int t = 0; t < XL; ++t)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void *)(dst + t * 1024), 16, lv[t & 1],
                                                  t * 16 * K + c * kXRow, 0, 0);
 }
 
 // One chunk: refill stage `nxt` and set `wn` (used in the previous step) with chunk c_next, wait
 // for chunk c, decode and multiply.  `cur` and `nxt` differ: the reads need not wait for the refill.
-template <int FMT, int I, int J, int S>
+template <int FMT, int I, int J, int S, int XL>
 __device__ __forceinline__ void chunk_step(const uint8_t *__restrict__ cur, uint8_t *__restrict__ nxt, bool refill, rsrc_t rx,
                                            const int (&lv)[2], int K, const WAddr &A, const uint32_t *__restrict__ sz, int cpg, int c,
                                            int c_next, int fr, int h,
                                            const DecodeK &D, const float (&rs)[I][2], const WSet<FMT> (&w)[I], WSet<FMT> (&wn)[I], floatx16 (&tot)[I][J]) {
-    constexpr int kLoads = 4 * J + w_loads<FMT>() * I;
+    constexpr int kLoads = XL + w_loads<FMT>() * I;
+    const int xr = XL < 4 * J ? min(fr, 8 * XL - 1) : fr;  // a lane past the staged rows repeats the last
     wait_vm_fence<63>();  // the previous step's reads of `nxt` returned
     if (refill) {
-        issue_x<J>(rx, nxt, lv, K, c_next);
+        issue_x<XL>(rx, nxt, lv, K, c_next);
 #pragma unroll
         for (int i = 0; i < I; ++i) load_w<FMT>(A, i, c_next, cpg, wn[i]);
     }
@@ -240,7 +242,7 @@ __device__ __forceinline__ void chunk_step(const uint8_t *__restrict__ cur, uint
         bf16x8_t xf[J];
 #pragma unroll
         for (int j = 0; j < J; ++j)
-            xf[j] = *reinterpret_cast<const bf16x8_t *>(cur + (32 * j + fr) * kXRow + xswz(fr, piece_of<FMT>(kk, h)) * 16);
+            xf[j] = *reinterpret_cast<const bf16x8_t *>(cur + (32 * j + xr) * kXRow + xswz(xr, piece_of<FMT>(kk, h)) * 16);
         if constexpr (FMT == FMT_I4G32 && (kk & 1) == 0) {
             const int nib = 2 * (c & 3) + (kk >> 1);
 #pragma unroll
@@ -322,16 +324,16 @@ __constant__ float kNf4S[16] = {
 
 // LDS of a workgroup: the x rings and the tile's `groups` scales and zero points (INT4) or the decode
 // table (NF4), later the waves' partial tiles.
-template <int FMT, int I, int J, int NW, int S>
+template <int FMT, int I, int J, int NW, int S, int XL>
 constexpr int64_t lds_bytes(int64_t groups) {
-    const int64_t ring = NW * S * 32 * J * kXRow + (FMT == FMT_INT4 ? groups * 32 * I * 4 : FMT == FMT_NF4 ? 256 * kCopies * 8 : 0), sums = NW * 32 * J * (32 * I + 4) * 4;
+    const int64_t ring = NW * S * XL * 1024 + (FMT == FMT_INT4 ? groups * 32 * I * 4 : FMT == FMT_NF4 ? 256 * kCopies * 8 : 0), sums = NW * 32 * J * (32 * I + 4) * 4;
     return ring > sums ? ring : sums;
 }
 constexpr int64_t kLdsMax = 160 * 1024;
 
-template <int FMT, int I, int J, int NW, int S>
+template <int FMT, int I, int J, int NW, int S, int XL>
 __global__ __launch_bounds__(64 * NW) void qsplit_kernel(QsArgs g) {
-    constexpr int kBN = 32 * I, kBM = 32 * J, kStage = kBM * kXRow;
+    constexpr int kBN = 32 * I, kBM = 32 * J, kStage = XL * 1024;
     extern __shared__ __align__(16) uint8_t lds[];
     // each XCD owns a contiguous run of tiles, in groups of up to 8 m tiles of one W panel (their x
     // rows stay in the XCD's L2)
@@ -414,7 +416,7 @@ __global__ __launch_bounds__(64 * NW) void qsplit_kernel(QsArgs g) {
         constexpr int t = decltype(TI)::value;
         if (t < n_own) {
             asm volatile("" ::: "memory");  // the waits count whole chunks
-            issue_x<J>(rx, ring + t * kStage, lv, K, c_of(t));
+            issue_x<XL>(rx, ring + t * kStage, lv, K, c_of(t));
 #pragma unroll
             for (int i = 0; i < I; ++i) load_w<FMT>(A, i, c_of(t), cpg, ws[t][i]);
         }
@@ -449,7 +451,7 @@ __global__ __launch_bounds__(64 * NW) void qsplit_kernel(QsArgs g) {
     for (; t0 + 2 * S - 2 < n_own; t0 += S)
         static_for<S>([&](auto SI) {
             constexpr int s = decltype(SI)::value, p = (s + S - 1) % S;
-            chunk_step<FMT, I, J, S>(ring + s * kStage, ring + p * kStage, true, rx, lv, K, A, sz, cpg, c_of(t0 + s),
+            chunk_step<FMT, I, J, S, XL>(ring + s * kStage, ring + p * kStage, true, rx, lv, K, A, sz, cpg, c_of(t0 + s),
                                      c_of(t0 + s + S - 1), fr, h, D, rs, ws[s], ws[p], tot);
         });
     for (; t0 < n_own; t0 += S)
@@ -458,7 +460,7 @@ __global__ __launch_bounds__(64 * NW) void qsplit_kernel(QsArgs g) {
             const int t = t0 + s;
             if (t < n_own) {
                 if (t + S - 1 >= n_own) wait_vm_fence<0>();  // fewer than S - 1 chunks follow
-                chunk_step<FMT, I, J, S>(ring + s * kStage, ring + p * kStage, t + S - 1 < n_own, rx, lv, K, A, sz, cpg,
+                chunk_step<FMT, I, J, S, XL>(ring + s * kStage, ring + p * kStage, t + S - 1 < n_own, rx, lv, K, A, sz, cpg,
                                          c_of(t), c_of(t + S - 1), fr, h, D, rs, ws[s], ws[p], tot);
             }
         });
@@ -511,12 +513,12 @@ __global__ __launch_bounds__(64 * NW) void qsplit_kernel(QsArgs g) {
 
 int64_t int4_groups(const QsProb &p) { return p.K / p.group; }
 
-template <int FMT, int I, int J, int NW, int S>
-void launch(QsArgs a, hipStream_t st) {
+template <int FMT, int I, int J, int NW, int S, int XL>
+void launch_x(QsArgs a, hipStream_t st) {
     int64_t lds = 0, tiles = 0;
     a.tiles_m = (a.M + 32 * J - 1) / (32 * J);
     for (int i = 0; i < a.count; ++i) {
-        lds = std::max(lds, lds_bytes<FMT, I, J, NW, S>(FMT == FMT_INT4 ? int4_groups(a.p[i]) : 0));
+        lds = std::max(lds, lds_bytes<FMT, I, J, NW, S, XL>(FMT == FMT_INT4 ? int4_groups(a.p[i]) : 0));
         a.p[i].tile_begin = static_cast<int>(tiles);
         tiles += static_cast<int64_t>(a.tiles_m) * ((a.p[i].N + 32 * I - 1) / (32 * I));
     }
@@ -526,7 +528,7 @@ void launch(QsArgs a, hipStream_t st) {
     int dev = 0;
     check_hip(hipGetDevice(&dev), "hipGetDevice");
     const uint64_t bit = dev < 64 ? (uint64_t{1} << dev) : 0;
-    const auto kern = qsplit_kernel<FMT, I, J, NW, S>;
+    const auto kern = qsplit_kernel<FMT, I, J, NW, S, XL>;
     if (bit == 0 || !(done.load(std::memory_order_acquire) & bit)) {
         check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMax),
                   "hipFuncSetAttribute(qsplit_kernel)");
@@ -536,8 +538,19 @@ void launch(QsArgs a, hipStream_t st) {
     check_launch("qsplit_kernel");
 }
 
+template <int FMT, int I, int J, int NW, int S>
+void launch(const QsArgs &a, hipStream_t st) {
+    if constexpr (J == 1) {
+        if (a.M <= 8) launch_x<FMT, I, J, NW, S, 1>(a, st);
+        else if (a.M <= 16) launch_x<FMT, I, J, NW, S, 2>(a, st);
+        else launch_x<FMT, I, J, NW, S, 4>(a, st);
+    } else {
+        launch_x<FMT, I, J, NW, S, 4 * J>(a, st);
+    }
+}
+
 // The tile by the number of workgroups (us per round of 256 workgroups at K = 4096, INT4 / INT8 /
-// Q8_0): 32 x 32 where M <= 32 or at most one tile per CU (8 / 9 / 11); 32 (n) x 64 up to one per CU
+// Q8_0): 32 x 32 up to one tile per CU, two for M <= 32 (8 / 9 / 11); 32 (n) x 64 up to one per CU
 // (12 / 12 / 14); then 64 x 64 (18 / 18 / 23 a round) or, above M = 64, 64 (n) x 128 (35 / 28 / 40)
 // where its rounds cost less.  Every shape up to M = 64 sums the same chunks in the same order, so a
 // batch gives the bits of one call per problem.
@@ -554,7 +567,13 @@ bool launch_fmt(const QsArgs &a, double r128, double rpf, hipStream_t st) {
     };
     const auto rounds = [&](int64_t t) { return static_cast<double>((t + cus - 1) / cus); };
     if (a.M <= 64) {
-        if (a.M <= 32 || tiles(32, 32) <= cus) launch<FMT_SMALL, 1, 1, 8, 2>(a, st);
+        // Beyond two 32 x 32 tiles per CU the decode's VALU time decides, and the skinny kernel's packed f16
+        // decode is half of this one's: the seven matrices of a 7B layer at M = 8, us there / here, INT4 48 /
+        // 55, INT8 56 / 84; M = 24 INT4 75 / 70, INT8 77 / 95; M = 64 141 / 94, 132 / 128.  (INT8 single calls
+        // above 32 rows would run the prefill kernel, which is slower.)
+        if (a.M <= (FMT == FMT_INT4 ? 16 : FMT == FMT_INT8 ? (a.count > 1 ? 48 : 32) : 0) && tiles(32, 32) > 2 * cus) return false;
+        if (tiles(32, 32) <= (a.M <= 32 ? 2 * cus : cus)) launch<FMT_SMALL, 1, 1, 8, 2>(a, st);
+        else if (a.M <= 32) launch<FMT_SMALL, 2, 1, 8, 2>(a, st);
         else if (tiles(32, 64) <= cus) launch<FMT_SMALL, 1, 2, 8, 2>(a, st);
         else launch<FMT_SMALL, 2, 2, 8, 2>(a, st);
         return true;
@@ -576,28 +595,28 @@ bool launch_fmt(const QsArgs &a, double r128, double rpf, hipStream_t st) {
 
 // NF4 (two MFMAs per product), us per round of 256 workgroups at K = 4096: 32 x 32 tiles up to one per CU
 // (10), 64 (n) x 32 beyond for M <= 32 (16), 32 (n) x 64 up to one per CU (14), then 64 x 64 (23 a round),
-// which holds to the largest M (4096 x 4096 at M = 512 / 4096: 49 / 322 us; the kernel of 128 (n) x 64 tiles
-// over two or four K parts that served M > 16 before took 36 at M = 64, 49 and 326, and 997 against 766
-// for 4096 x 11008 at M = 4096).  All sum the same chunks in the same order.
-void launch_nf4(const QsArgs &a, hipStream_t st) {
+// which holds to the largest M (4096 x 4096 at M = 64 / 512 / 4096 12 / 49 / 322 us, nf4_mfma_kernel 36 /
+// 49 / 326; 4096 x 11008 at M = 4096 766 / 997).  All sum the same chunks in the same order.
+// False for M <= 64 with more than one 64 x 64 tile per CU, where nf4_mfma_kernel's cheaper decode decides
+// (the seven matrices of a 7B layer at M = 64: 85 us there, 122 here).
+bool launch_nf4(const QsArgs &a, hipStream_t st) {
     const int64_t cus = cu_count();
     const auto tiles = [&](int64_t bn, int64_t bm) {
         int64_t t = 0;
         for (int i = 0; i < a.count; ++i) t += (a.M + bm - 1) / bm * ((a.p[i].N + bn - 1) / bn);
         return t;
     };
+    if (a.M <= 64 && tiles(64, 64) > cus) return false;
     if (tiles(32, 32) <= cus) launch<FMT_NF4, 1, 1, 8, 2>(a, st);
     else if (a.M <= 32) launch<FMT_NF4, 2, 1, 8, 2>(a, st);
     else if (tiles(32, 64) <= cus) launch<FMT_NF4, 1, 2, 8, 2>(a, st);
     else launch<FMT_NF4, 2, 2, 8, 2>(a, st);
+    return true;
 }
 
 bool launch_any(int fmt, const QsArgs &a, hipStream_t st) {
     if (fmt == FMT_INT8) return launch_fmt<FMT_INT8, FMT_I8S>(a, 1.5, 3.1, st);
-    if (fmt == FMT_NF4) {
-        launch_nf4(a, st);
-        return true;
-    }
+    if (fmt == FMT_NF4) return launch_nf4(a, st);
     if (fmt == FMT_Q4G) return launch_fmt<FMT_Q4G, FMT_Q4G>(a, 1.75, 4.0, st);
     if (fmt == FMT_Q8G) return launch_fmt<FMT_Q8G, FMT_Q8G>(a, 1.75, 4.6, st);
     if (a.p[0].group == 32) return launch_fmt<FMT_I4G32, FMT_I4G32>(a, 1.65, 3.5, st);
@@ -616,6 +635,9 @@ QsProb prob(const uint16_t *x, int64_t n, int64_t k, int64_t group, const void *
 // kernel keep M > 16 off it.
 bool qsplit_ok(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes, const void *scales) {
     if (fmt != FMT_INT4 && fmt != FMT_INT8 && fmt != FMT_NF4 && fmt != FMT_Q4G && fmt != FMT_Q8G) return false;
+    // GGUF up to 32 rows: the skinny kernel, for single calls too, so that a batch gives their bits (a layer's
+    // seven Q8_0 matrices in one launch at M = 8: 69 us there, 110 here; one 4096 x 4096 13 / 10)
+    if ((fmt == FMT_Q4G || fmt == FMT_Q8G) && m <= 32) return false;
     // NF4: M > 16 (a partial reaches 64 |x|; up to 16 rows the skinny kernels take any finite x), blocks a
     // power of two; CASTFORGE_NF4_MFMA=0 keeps it on the skinny / prefill kernels (for comparison)
     if (fmt == FMT_NF4) {
@@ -633,7 +655,7 @@ bool qsplit_ok(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int6
     if (fmt == FMT_INT4) {
         if (k % group != 0 || (group != 32 && group % kChunk != 0)) return false;
         // groups of 64 and more: the largest tile's scales and zero points next to the x rings
-        if (group != 32 && lds_bytes<FMT_INT4, 2, 2, 8, 2>(k / group) > kLdsMax) return false;
+        if (group != 32 && lds_bytes<FMT_INT4, 2, 2, 8, 2, 8>(k / group) > kLdsMax) return false;
     }
     if (fmt != FMT_NF4 && m > 16 && (std::getenv("CASTFORGE_PREFILL_I4") || std::getenv("CASTFORGE_PREFILL_TILE"))) return false;
     return true;
@@ -650,8 +672,9 @@ bool qsplit_try(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int
 }
 
 // One launch over up to CFH_MAX_BATCH INT8 / INT4 / NF4 / GGUF problems of one format and group (INT4:
-// whole multiples of 64) with the same M (2..64), each checked by qsplit_ok.
-void qsplit_batch(int fmt, int64_t m, int count, const uint16_t *const *x, const int64_t *n, const int64_t *k,
+// whole multiples of 64) with the same M (2..64), each checked by qsplit_ok; false where another kernel is
+// faster for as many tiles.
+bool qsplit_batch(int fmt, int64_t m, int count, const uint16_t *const *x, const int64_t *n, const int64_t *k,
                   const int64_t *group, const void *const *codes, const void *const *scales, const uint32_t *const *zeros,
                   const int *per_row, void *const *y, int y_bf16, hipStream_t st) {
     require(count >= 1 && count <= CFH_MAX_BATCH && m >= 2 && m <= 64, "qsplit_batch: 1..CFH_MAX_BATCH problems, M = 2..64");
@@ -665,7 +688,7 @@ void qsplit_batch(int fmt, int64_t m, int count, const uint16_t *const *x, const
         a.p[i] = prob(x[o], n[o], k[o], group[o], codes[o], scales[o], zeros[o], per_row[o], y[o]);
     }
     a.count = count, a.M = static_cast<int>(m), a.y_bf16 = y_bf16;
-    require(launch_any(fmt, a, st), "qsplit_batch: no tile");
+    return launch_any(fmt, a, st);
 }
 
 }  // namespace cfh

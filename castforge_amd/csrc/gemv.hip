@@ -1623,12 +1623,23 @@ bool prefill_try(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, in
 bool qsplit_try(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes,
                 const void *scales, const uint32_t *zeros, int per_row, void *y, int y_bf16, hipStream_t st);
 bool qsplit_ok(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes, const void *scales);
-void qsplit_batch(int fmt, int64_t m, int count, const uint16_t *const *x, const int64_t *n, const int64_t *k,
+bool qsplit_batch(int fmt, int64_t m, int count, const uint16_t *const *x, const int64_t *n, const int64_t *k,
                   const int64_t *group, const void *const *codes, const void *const *scales, const uint32_t *const *zeros,
                   const int *per_row, void *const *y, int y_bf16, hipStream_t st);
 
+// NF4 on one bf16 MFMA pair per product (gemm_nf4.hip), for M > 16.
+bool nf4_mfma_ok(const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t block, const void *codes);
+void nf4_mfma_launch(const cfh_nf4_problem_t *ps, int count, int64_t m, int y_bf16, hipStream_t st);
+
+// CASTFORGE_NF4_MFMA=0 keeps NF4 at M > 16 on the skinny / prefill kernels (for comparison).
+bool nf4_mfma_enabled() {
+    const char *e = std::getenv("CASTFORGE_NF4_MFMA");
+    return !(e && std::strcmp(e, "0") == 0);
+}
+
 // A batch (each problem passes skinny_ok): the problems that qsplit_kernel takes in one launch of
-// it, as single calls do, the others in one launch of the skinny kernels.
+// it where their tiles are few, the others in one launch of nf4_mfma_kernel (NF4 at M > 16) or of the
+// skinny kernels.
 void launch_batch(int fmt, Problem *ps, int count, int64_t m, int y_bf16, hipStream_t st) {
     const uint16_t *x[kMaxProblems];
     int64_t n[kMaxProblems], k[kMaxProblems], group[kMaxProblems];
@@ -1636,19 +1647,32 @@ void launch_batch(int fmt, Problem *ps, int count, int64_t m, int y_bf16, hipStr
     const uint32_t *zeros[kMaxProblems];
     int per_row[kMaxProblems];
     void *y[kMaxProblems];
+    Problem others[kMaxProblems];
     int used = 0, rest = 0;
     for (int i = 0; i < count; ++i) {
-        const Problem p = ps[i];
+        const Problem &p = ps[i];
         if (!qsplit_ok(fmt, p.x, m, p.n, p.k, p.group, p.codes, p.scales)) {
-            ps[rest++] = p;
+            others[rest++] = p;
             continue;
         }
         x[used] = p.x, n[used] = p.n, k[used] = p.k, group[used] = p.group, codes[used] = p.codes, scales[used] = p.scales;
         zeros[used] = p.zeros, per_row[used] = p.scale_per_row, y[used] = p.y;
         ++used;
     }
-    if (used) qsplit_batch(fmt, m, used, x, n, k, group, codes, scales, zeros, per_row, y, y_bf16, st);
-    if (rest) launch_skinny(fmt, ps, rest, m, y_bf16, st);
+    if (used && !qsplit_batch(fmt, m, used, x, n, k, group, codes, scales, zeros, per_row, y, y_bf16, st)) {
+        rest = count;
+        std::copy(ps, ps + count, others);
+    }
+    if (rest == 0) return;
+    bool mfma = fmt == FMT_NF4 && nf4_mfma_enabled();
+    cfh_nf4_problem_t mf[kMaxProblems];
+    for (int i = 0; i < rest && mfma; ++i) {
+        const Problem &p = others[i];
+        mfma = nf4_mfma_ok(p.x, m, p.n, p.k, p.group, p.codes);
+        mf[i] = {p.x, static_cast<const uint32_t *>(p.codes), static_cast<const float *>(p.scales), p.y, p.n, p.k, p.group};
+    }
+    if (mfma) nf4_mfma_launch(mf, rest, m, y_bf16, st);
+    else launch_skinny(fmt, others, rest, m, y_bf16, st);
 }
 
 // Largest M a single problem runs on the skinny kernels; beyond it the prefill kernel is
@@ -1731,8 +1755,13 @@ int32_t castforge_hip_gemv_nf4(const uint16_t *x, int64_t m, int64_t n, int64_t 
         require(k == 0 || absmax, "absmax must not be NULL");
         hipStream_t st = static_cast<hipStream_t>(stream);
         const int yb = y_dtype == CFH_DTYPE_BF16;
-        if (!qsplit_try(FMT_NF4, x, m, n, k, block, codes, absmax, nullptr, 1, y, yb, st) &&
-            !gemv_try_skinny(FMT_NF4, x, m, n, k, block, codes, absmax, nullptr, 1, y, yb, st) &&
+        if (qsplit_try(FMT_NF4, x, m, n, k, block, codes, absmax, nullptr, 1, y, yb, st)) return;
+        if (nf4_mfma_enabled() && nf4_mfma_ok(x, m, n, k, block, codes)) {
+            const cfh_nf4_problem_t p{x, codes, absmax, y, n, k, block};
+            nf4_mfma_launch(&p, 1, m, yb, st);
+            return;
+        }
+        if (!gemv_try_skinny(FMT_NF4, x, m, n, k, block, codes, absmax, nullptr, 1, y, yb, st) &&
             !prefill_try(FMT_NF4, x, m, n, k, block, codes, absmax, nullptr, 1, y, yb, st))
             gemv_generic(FMT_NF4, x, m, n, k, block, codes, absmax, nullptr, 1, y, yb, st);
     });

@@ -56,7 +56,7 @@ def test_split_vs_float64(cuda, fmt, k, m, n):
     # (batched INT4 takes groups of 128; a single GGUF call of two rows runs the M = 1 kernel)
     if m <= 64 and (fmt in ("int4_128", "int8_channel", "int8_tensor") or fmt[0] == "n" or m > 2 and fmt[0] == "q"):
         yy = torch.empty_like(y)
-        run_batched(x, yy)
+        run_batched(x, yy)  # one problem: by the same rule as the single call
         assert torch.equal(yy, y)
 
 
