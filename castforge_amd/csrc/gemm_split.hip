@@ -335,17 +335,19 @@ template <int FMT, int I, int J, int NW, int S, int XL>
 __global__ __launch_bounds__(64 * NW) void qsplit_kernel(QsArgs g) {
     constexpr int kBN = 32 * I, kBM = 32 * J, kStage = XL * 1024;
     extern __shared__ __align__(16) uint8_t lds[];
-    // each XCD owns a contiguous run of tiles, in groups of up to 8 m tiles of one W panel (their x
-    // rows stay in the XCD's L2)
-    int pid = blockIdx.x;
-    {
-        const int per_xcd = g.tiles / kXcds, full = per_xcd * kXcds;
-        if (pid < full) pid = (pid % kXcds) * per_xcd + pid / kXcds;
-    }
-    int pi = 0;
+    int pid = blockIdx.x, pi = 0;
     while (pi + 1 < g.count && pid >= g.p[pi + 1].tile_begin) ++pi;
     const QsProb &a = g.p[pi];
     pid -= a.tile_begin;
+    // each XCD owns a contiguous run of each problem's tiles, in groups of up to 8 m tiles of one W panel
+    // (their x rows stay in the XCD's L2).  A run of the whole batch's tiles instead, longest K first, gave one
+    // XCD all of a layer's W_down (the seven matrices, us, whole batch / each problem: INT4 at M = 8 54 / 37,
+    // INT8 87 / 61; Q8_0 at M = 40 143 / 93; NF4 at M = 64 122 / 71).
+    {
+        const int tiles = (pi + 1 < g.count ? g.p[pi + 1].tile_begin : g.tiles) - a.tile_begin;
+        const int per_xcd = tiles / kXcds, full = per_xcd * kXcds;
+        if (pid < full) pid = (pid % kXcds) * per_xcd + pid / kXcds;
+    }
     const int M = g.M, N = a.N, K = a.K;
     const int tiles_n = (N + kBN - 1) / kBN;
     const int span = 8 * tiles_n, first_m = pid / span * 8, gm = min(8, g.tiles_m - first_m);
