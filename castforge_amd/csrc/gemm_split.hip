@@ -551,78 +551,86 @@ void launch(const QsArgs &a, hipStream_t st) {
     }
 }
 
+int64_t tiles_of(const QsArgs &a, int64_t bn, int64_t bm) {
+    int64_t t = 0;
+    for (int i = 0; i < a.count; ++i) t += (a.M + bm - 1) / bm * ((a.p[i].N + bn - 1) / bn);
+    return t;
+}
+double rounds(int64_t tiles) { return static_cast<double>((tiles + cu_count() - 1) / cu_count()); }
+
+// Rounds of 64 x 64 tiles that a round of 64 (n) x 128 takes the time of, and that a round of the one-MFMA
+// prefill kernel's 256 (n) x 128 tiles takes, however few they are.
+struct Costs {
+    double r128, rpf;
+};
+Costs costs(int fmt, int64_t group) {
+    if (fmt == FMT_INT8) return {1.5, 3.1};
+    if (fmt == FMT_Q4G) return {1.75, 4.0};
+    if (fmt == FMT_Q8G) return {1.75, 4.6};
+    return group == 32 ? Costs{1.65, 3.5} : Costs{1.95, 4.0};
+}
+
+// Whether a problem of the kernel's runs on it.  By the problem alone, so that a batch gives the bits of
+// one call per problem:
+//   * up to 64 rows always; NF4 up to one 64 x 64 tile per CU, beyond which nf4_mfma_kernel's cheaper decode
+//     decides (K = 4096 at M = 17 / 64, us there / here: n = 16384 27.7 / 17.2, 37 / 25; n = 17000 27.6 /
+//     29.3, 37 / 42);
+//   * above, where the one-MFMA prefill kernel does not cost less (INT4, 4096 x 4096 at M = 512: 33 us here
+//     against 59; 11008 x 4096 at M = 512: 92 against 68; 4096 x 11008 at M = 603: 104 against 123); NF4 always.
+bool chosen(int fmt, const QsArgs &a) {
+    if (fmt == FMT_NF4) return a.M > 64 || tiles_of(a, 64, 64) <= cu_count();
+    if (a.M <= 64 || tiles_of(a, 32, 64) <= cu_count()) return true;
+    const Costs c = costs(fmt, a.p[0].group);
+    const double here = std::min(rounds(tiles_of(a, 64, 64)), c.r128 * rounds(tiles_of(a, 64, 128)));
+    const bool rows96 = fmt != FMT_INT8 && (fmt != FMT_INT4 || (a.p[0].group != 64 && a.p[0].group != 32));
+    return here <= c.rpf * prefill_cost(fmt, rows96, a.M, a.p[0].N);
+}
+
 // The tile by the number of workgroups (us per round of 256 workgroups at K = 4096, INT4 / INT8 /
-// Q8_0): 32 x 32 up to one tile per CU, two for M <= 32 (8 / 9 / 11); 32 (n) x 64 up to one per CU
-// (12 / 12 / 14); then 64 x 64 (18 / 18 / 23 a round) or, above M = 64, 64 (n) x 128 (35 / 28 / 40)
-// where its rounds cost less.  Every shape up to M = 64 sums the same chunks in the same order, so a
-// batch gives the bits of one call per problem.
-// False (M > 64) where the one-MFMA prefill kernel costs less still: a round of its 256 (n) x 128
-// tiles takes rpf rounds of 64 x 64 however few its tiles (INT4, 4096 x 4096 at M = 512: 33 us here
-// against 59; 11008 x 4096 at M = 512: 92 against 68; 4096 x 11008 at M = 603: 104 against 123).
+// Q8_0): 32 x 32 up to one tile per CU (8 / 9 / 11), three for M <= 32 (n = 20000, 625 tiles, at M = 8
+// 16.9 / 24.0; as 64 x 32 20.0 / 32.1), INT8 at M <= 16 always (the per-row form decodes twice as long:
+// n = 131072 119 against 136); then 64 (n) x 32 for M <= 32 (INT4 n = 32000 at M = 24 26.0; as 32 x 32
+// 29.7); 32 (n) x 64 up to one per CU (12 / 12 / 14); then 64 x 64 (18 / 18 / 23 a round) or, above
+// M = 64, 64 (n) x 128 (35 / 28 / 40) where its rounds cost less.  Every shape up to M = 64 sums the same
+// chunks in the same order.
 template <int FMT, int FMT_SMALL>
-bool launch_fmt(const QsArgs &a, double r128, double rpf, hipStream_t st) {
-    const int64_t cus = cu_count();
-    const auto tiles = [&](int64_t bn, int64_t bm) {
-        int64_t t = 0;
-        for (int i = 0; i < a.count; ++i) t += (a.M + bm - 1) / bm * ((a.p[i].N + bn - 1) / bn);
-        return t;
-    };
-    const auto rounds = [&](int64_t t) { return static_cast<double>((t + cus - 1) / cus); };
-    if (a.M <= 64) {
-        // Beyond two 32 x 32 tiles per CU the decode's VALU time decides, and the skinny kernel's packed f16
-        // decode is half of this one's: the seven matrices of a 7B layer at M = 8, us there / here, INT4 48 /
-        // 55, INT8 56 / 84; M = 24 INT4 75 / 70, INT8 77 / 95; M = 64 141 / 94, 132 / 128.  (INT8 single calls
-        // above 32 rows would run the prefill kernel, which is slower.)
-        if (a.M <= (FMT == FMT_INT4 ? 16 : FMT == FMT_INT8 ? (a.count > 1 ? 48 : 32) : 0) && tiles(32, 32) > 2 * cus) return false;
-        if (tiles(32, 32) <= (a.M <= 32 ? 2 * cus : cus)) launch<FMT_SMALL, 1, 1, 8, 2>(a, st);
-        else if (a.M <= 32) launch<FMT_SMALL, 2, 1, 8, 2>(a, st);
-        else if (tiles(32, 64) <= cus) launch<FMT_SMALL, 1, 2, 8, 2>(a, st);
-        else launch<FMT_SMALL, 2, 2, 8, 2>(a, st);
-        return true;
-    }
-    if (tiles(32, 32) <= cus) {
+void launch_fmt(const QsArgs &a, hipStream_t st) {
+    const int64_t cus = cu_count(), t32 = tiles_of(a, 32, 32);
+    if (t32 <= (a.M <= 32 ? 3 * cus : cus) || (FMT == FMT_INT8 && a.M <= 16)) {
         launch<FMT_SMALL, 1, 1, 8, 2>(a, st);
-        return true;
-    }
-    if (tiles(32, 64) <= cus) {
+    } else if (a.M <= 32) {
+        launch<FMT_SMALL, 2, 1, 8, 2>(a, st);
+    } else if (a.M <= 64) {
+        if (tiles_of(a, 32, 64) <= cus) launch<FMT_SMALL, 1, 2, 8, 2>(a, st);
+        else launch<FMT_SMALL, 2, 2, 8, 2>(a, st);
+    } else if (tiles_of(a, 32, 64) <= cus) {
         launch<FMT, 1, 2, 8, 2>(a, st);
-        return true;
+    } else if (rounds(tiles_of(a, 64, 64)) <= costs(FMT == FMT_I4G32 ? FMT_INT4 : FMT, a.p[0].group).r128 * rounds(tiles_of(a, 64, 128))) {
+        launch<FMT, 2, 2, 8, 2>(a, st);
+    } else {
+        launch<FMT, 2, 4, 4, 2>(a, st);
     }
-    const double c64 = rounds(tiles(64, 64)), c128 = r128 * rounds(tiles(64, 128));
-    if (std::min(c64, c128) > rpf * prefill_cost(FMT, FMT != FMT_INT8 && a.p[0].group != 64 && FMT != FMT_I4G32, a.M, a.p[0].N)) return false;
-    if (c64 <= c128) launch<FMT, 2, 2, 8, 2>(a, st);
-    else launch<FMT, 2, 4, 4, 2>(a, st);
-    return true;
 }
 
 // NF4 (two MFMAs per product), us per round of 256 workgroups at K = 4096: 32 x 32 tiles up to one per CU
 // (10), 64 (n) x 32 beyond for M <= 32 (16), 32 (n) x 64 up to one per CU (14), then 64 x 64 (23 a round),
 // which holds to the largest M (4096 x 4096 at M = 64 / 512 / 4096 12 / 49 / 322 us, nf4_mfma_kernel 36 /
 // 49 / 326; 4096 x 11008 at M = 4096 766 / 997).  All sum the same chunks in the same order.
-// False for M <= 64 with more than one 64 x 64 tile per CU, where nf4_mfma_kernel's cheaper decode decides
-// (the seven matrices of a 7B layer at M = 64: 85 us there, 122 here).
-bool launch_nf4(const QsArgs &a, hipStream_t st) {
+void launch_nf4(const QsArgs &a, hipStream_t st) {
     const int64_t cus = cu_count();
-    const auto tiles = [&](int64_t bn, int64_t bm) {
-        int64_t t = 0;
-        for (int i = 0; i < a.count; ++i) t += (a.M + bm - 1) / bm * ((a.p[i].N + bn - 1) / bn);
-        return t;
-    };
-    if (a.M <= 64 && tiles(64, 64) > cus) return false;
-    if (tiles(32, 32) <= cus) launch<FMT_NF4, 1, 1, 8, 2>(a, st);
+    if (tiles_of(a, 32, 32) <= cus) launch<FMT_NF4, 1, 1, 8, 2>(a, st);
     else if (a.M <= 32) launch<FMT_NF4, 2, 1, 8, 2>(a, st);
-    else if (tiles(32, 64) <= cus) launch<FMT_NF4, 1, 2, 8, 2>(a, st);
+    else if (tiles_of(a, 32, 64) <= cus) launch<FMT_NF4, 1, 2, 8, 2>(a, st);
     else launch<FMT_NF4, 2, 2, 8, 2>(a, st);
-    return true;
 }
 
-bool launch_any(int fmt, const QsArgs &a, hipStream_t st) {
-    if (fmt == FMT_INT8) return launch_fmt<FMT_INT8, FMT_I8S>(a, 1.5, 3.1, st);
-    if (fmt == FMT_NF4) return launch_nf4(a, st);
-    if (fmt == FMT_Q4G) return launch_fmt<FMT_Q4G, FMT_Q4G>(a, 1.75, 4.0, st);
-    if (fmt == FMT_Q8G) return launch_fmt<FMT_Q8G, FMT_Q8G>(a, 1.75, 4.6, st);
-    if (a.p[0].group == 32) return launch_fmt<FMT_I4G32, FMT_I4G32>(a, 1.65, 3.5, st);
-    return launch_fmt<FMT_INT4, FMT_INT4>(a, 1.95, 4.0, st);
+void launch_any(int fmt, const QsArgs &a, hipStream_t st) {
+    if (fmt == FMT_INT8) launch_fmt<FMT_INT8, FMT_I8S>(a, st);
+    else if (fmt == FMT_NF4) launch_nf4(a, st);
+    else if (fmt == FMT_Q4G) launch_fmt<FMT_Q4G, FMT_Q4G>(a, st);
+    else if (fmt == FMT_Q8G) launch_fmt<FMT_Q8G, FMT_Q8G>(a, st);
+    else if (a.p[0].group == 32) launch_fmt<FMT_I4G32, FMT_I4G32>(a, st);
+    else launch_fmt<FMT_INT4, FMT_INT4>(a, st);
 }
 
 QsProb prob(const uint16_t *x, int64_t n, int64_t k, int64_t group, const void *codes, const void *scales,
@@ -637,8 +645,9 @@ QsProb prob(const uint16_t *x, int64_t n, int64_t k, int64_t group, const void *
 // kernel keep M > 16 off it.
 bool qsplit_ok(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes, const void *scales) {
     if (fmt != FMT_INT4 && fmt != FMT_INT8 && fmt != FMT_NF4 && fmt != FMT_Q4G && fmt != FMT_Q8G) return false;
-    // GGUF up to 32 rows: the skinny kernel, for single calls too, so that a batch gives their bits (a layer's
-    // seven Q8_0 matrices in one launch at M = 8: 69 us there, 110 here; one 4096 x 4096 13 / 10)
+    // GGUF up to 32 rows: the skinny kernel, for single calls too, so that a batch gives their bits (Q8_0 / Q4_0
+    // at M = 8, us there / here: W_gate and W_up in one launch 36 / 41, 26 / 34; a layer's seven matrices 71 / 75,
+    // 50 / 59; one 4096 x 4096 14 / 11, 11 / 10)
     if ((fmt == FMT_Q4G || fmt == FMT_Q8G) && m <= 32) return false;
     // NF4: M > 16 (a partial reaches 64 |x|; up to 16 rows the skinny kernels take any finite x), blocks a
     // power of two; CASTFORGE_NF4_MFMA=0 keeps it on the skinny / prefill kernels (for comparison)
@@ -663,20 +672,29 @@ bool qsplit_ok(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int6
     return true;
 }
 
+// Whether qsplit_kernel runs a problem, alone or in a batch.
+bool qsplit_takes(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes, const void *scales) {
+    if (!qsplit_ok(fmt, x, m, n, k, group, codes, scales)) return false;
+    QsArgs a{};
+    a.p[0].N = static_cast<int>(n), a.p[0].K = static_cast<int>(k), a.p[0].group = static_cast<int>(group);
+    a.count = 1, a.M = static_cast<int>(m);
+    return chosen(fmt, a);
+}
+
 // Runs a product on qsplit_kernel; false where the kernel does not take it or another is faster.
 bool qsplit_try(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes,
                 const void *scales, const uint32_t *zeros, int per_row, void *y, int y_bf16, hipStream_t st) {
-    if (!qsplit_ok(fmt, x, m, n, k, group, codes, scales)) return false;
+    if (!qsplit_takes(fmt, x, m, n, k, group, codes, scales)) return false;
     QsArgs a{};
     a.p[0] = prob(x, n, k, group, codes, scales, zeros, per_row, y);
     a.count = 1, a.M = static_cast<int>(m), a.y_bf16 = y_bf16;
-    return launch_any(fmt, a, st);
+    launch_any(fmt, a, st);
+    return true;
 }
 
 // One launch over up to CFH_MAX_BATCH INT8 / INT4 / NF4 / GGUF problems of one format and group (INT4:
-// whole multiples of 64) with the same M (2..64), each checked by qsplit_ok; false where another kernel is
-// faster for as many tiles.
-bool qsplit_batch(int fmt, int64_t m, int count, const uint16_t *const *x, const int64_t *n, const int64_t *k,
+// whole multiples of 64) with the same M (2..64), each one that qsplit_takes.
+void qsplit_batch(int fmt, int64_t m, int count, const uint16_t *const *x, const int64_t *n, const int64_t *k,
                   const int64_t *group, const void *const *codes, const void *const *scales, const uint32_t *const *zeros,
                   const int *per_row, void *const *y, int y_bf16, hipStream_t st) {
     require(count >= 1 && count <= CFH_MAX_BATCH && m >= 2 && m <= 64, "qsplit_batch: 1..CFH_MAX_BATCH problems, M = 2..64");
@@ -690,7 +708,7 @@ bool qsplit_batch(int fmt, int64_t m, int count, const uint16_t *const *x, const
         a.p[i] = prob(x[o], n[o], k[o], group[o], codes[o], scales[o], zeros[o], per_row[o], y[o]);
     }
     a.count = count, a.M = static_cast<int>(m), a.y_bf16 = y_bf16;
-    return launch_any(fmt, a, st);
+    launch_any(fmt, a, st);
 }
 
 }  // namespace cfh

@@ -1622,8 +1622,8 @@ bool prefill_try(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, in
 // K split over a workgroup's waves (gemm_split.hip); false where it does not take the problem.
 bool qsplit_try(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes,
                 const void *scales, const uint32_t *zeros, int per_row, void *y, int y_bf16, hipStream_t st);
-bool qsplit_ok(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes, const void *scales);
-bool qsplit_batch(int fmt, int64_t m, int count, const uint16_t *const *x, const int64_t *n, const int64_t *k,
+bool qsplit_takes(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes, const void *scales);
+void qsplit_batch(int fmt, int64_t m, int count, const uint16_t *const *x, const int64_t *n, const int64_t *k,
                   const int64_t *group, const void *const *codes, const void *const *scales, const uint32_t *const *zeros,
                   const int *per_row, void *const *y, int y_bf16, hipStream_t st);
 
@@ -1637,9 +1637,10 @@ bool nf4_mfma_enabled() {
     return !(e && std::strcmp(e, "0") == 0);
 }
 
-// A batch (each problem passes skinny_ok): the problems that qsplit_kernel takes in one launch of
-// it where their tiles are few, the others in one launch of nf4_mfma_kernel (NF4 at M > 16) or of the
-// skinny kernels.
+// A batch (each problem passes skinny_ok): the problems that qsplit_kernel takes in one launch of it, the
+// others in one launch of nf4_mfma_kernel (NF4 at M > 16) or of the skinny kernels.  A problem runs on the
+// kernel of its single call whatever else is in the batch, and gives the same bits (but above M = 16 where
+// a single call would run a prefill kernel).
 void launch_batch(int fmt, Problem *ps, int count, int64_t m, int y_bf16, hipStream_t st) {
     const uint16_t *x[kMaxProblems];
     int64_t n[kMaxProblems], k[kMaxProblems], group[kMaxProblems];
@@ -1651,7 +1652,7 @@ void launch_batch(int fmt, Problem *ps, int count, int64_t m, int y_bf16, hipStr
     int used = 0, rest = 0;
     for (int i = 0; i < count; ++i) {
         const Problem &p = ps[i];
-        if (!qsplit_ok(fmt, p.x, m, p.n, p.k, p.group, p.codes, p.scales)) {
+        if (!qsplit_takes(fmt, p.x, m, p.n, p.k, p.group, p.codes, p.scales)) {
             others[rest++] = p;
             continue;
         }
@@ -1659,20 +1660,18 @@ void launch_batch(int fmt, Problem *ps, int count, int64_t m, int y_bf16, hipStr
         zeros[used] = p.zeros, per_row[used] = p.scale_per_row, y[used] = p.y;
         ++used;
     }
-    if (used && !qsplit_batch(fmt, m, used, x, n, k, group, codes, scales, zeros, per_row, y, y_bf16, st)) {
-        rest = count;
-        std::copy(ps, ps + count, others);
-    }
-    if (rest == 0) return;
-    bool mfma = fmt == FMT_NF4 && nf4_mfma_enabled();
+    if (used) qsplit_batch(fmt, m, used, x, n, k, group, codes, scales, zeros, per_row, y, y_bf16, st);
     cfh_nf4_problem_t mf[kMaxProblems];
-    for (int i = 0; i < rest && mfma; ++i) {
+    int mfma = 0, skinny = 0;
+    for (int i = 0; i < rest; ++i) {
         const Problem &p = others[i];
-        mfma = nf4_mfma_ok(p.x, m, p.n, p.k, p.group, p.codes);
-        mf[i] = {p.x, static_cast<const uint32_t *>(p.codes), static_cast<const float *>(p.scales), p.y, p.n, p.k, p.group};
+        if (fmt == FMT_NF4 && nf4_mfma_enabled() && nf4_mfma_ok(p.x, m, p.n, p.k, p.group, p.codes))
+            mf[mfma++] = {p.x, static_cast<const uint32_t *>(p.codes), static_cast<const float *>(p.scales), p.y, p.n, p.k, p.group};
+        else
+            others[skinny++] = p;
     }
-    if (mfma) nf4_mfma_launch(mf, rest, m, y_bf16, st);
-    else launch_skinny(fmt, others, rest, m, y_bf16, st);
+    if (mfma) nf4_mfma_launch(mf, mfma, m, y_bf16, st);
+    if (skinny) launch_skinny(fmt, others, skinny, m, y_bf16, st);
 }
 
 // Largest M a single problem runs on the skinny kernels; beyond it the prefill kernel is

@@ -14,24 +14,30 @@ SHAPES = [(2, 1), (31, 65), (19, 9000), (33, 64), (64, 97), (40, 4200), (70, 280
 
 
 def _weight(fmt, n, k, cuda):
+    wd, run, run_batch, p = _packed(fmt, n, k, cuda)
+    return wd, run, lambda x, y: run_batch([x], [p], [y])
+
+
+def _packed(fmt, n, k, cuda):
+    """Dequantized weight, single call (x, out dtype), batched call (xs, packed, ys), packed weight."""
     w = torch.from_numpy(synth.weight(31, n, n, k)).to(cuda)
     if fmt.startswith("int4"):
         p = ops.quantize_int4g(w, int(fmt[5:]))
-        return ops.dequantize_int4g(p), lambda x, o: ops.gemm_w4a16(x, p, o), lambda x, y: ops.gemv_w4a16_batched([x], [p], [y])
+        return ops.dequantize_int4g(p), lambda x, o: ops.gemm_w4a16(x, p, o), ops.gemv_w4a16_batched, p
     if fmt.startswith("int8"):
         gran = fmt[5:]
         q, s = ops.quantize_int8(w, 8, gran)
         return (ops.dequantize_int8(q, s, gran), lambda x, o: ops.gemm_w8a16(x, q, s, gran, o),
-                lambda x, y: ops.gemv_w8a16_batched([x], [(q, s)], [y], gran))
+                lambda xs, ps, ys: ops.gemv_w8a16_batched(xs, ps, ys, gran), (q, s))
     if fmt.startswith("nf4"):
         p = ops.quantize_nf4(w, int(fmt[4:]))
-        return ops.dequantize_nf4(p), lambda x, o: ops.gemm_nf4(x, p, o), lambda x, y: ops.gemv_nf4_batched([x], [p], [y])
+        return ops.dequantize_nf4(p), lambda x, o: ops.gemm_nf4(x, p, o), ops.gemv_nf4_batched, p
     ty, size = (ffi.GGML_Q4_0, 18) if fmt == "q4_0" else (ffi.GGML_Q8_0, 34)
     rng = np.random.default_rng(n + k)
     raw = rng.integers(0, 256, (n * k // 32, size), dtype=np.uint8)
     raw[:, :2] = rng.uniform(1e-3, 2e-3, (n * k // 32, 1)).astype(np.float16).view(np.uint8)
     p = ops.gguf_repack(ty, torch.from_numpy(raw.reshape(-1)).to(cuda), n, k)
-    return ops.dequantize_gguf(p), lambda x, o: ops.gemm_gguf(x, p, o), lambda x, y: ops.gemv_gguf_batched([x], [p], [y])
+    return ops.dequantize_gguf(p), lambda x, o: ops.gemm_gguf(x, p, o), ops.gemv_gguf_batched, p
 
 
 # k: fewer 64-wide chunks than the workgroup's eight waves, and 18 chunks (some waves one more)
@@ -58,6 +64,34 @@ def test_split_vs_float64(cuda, fmt, k, m, n):
         yy = torch.empty_like(y)
         run_batched(x, yy)  # one problem: by the same rule as the single call
         assert torch.equal(yy, y)
+
+
+# the seven projections of a decoder layer in n, short in k, two with remainders: more than three 32 x 32
+# tiles per CU, so that M <= 32 runs 64 (n) x 32 tiles where the format has them
+LAYER = [(4096, 256)] * 3 + [(4099, 384), (11008, 256), (11001, 256), (4096, 1152)]
+
+
+@pytest.mark.parametrize("fmt", ["int4_128", "int8_channel", "int8_tensor", "nf4_64", "q4_0", "q8_0"])
+def test_layer_batch_gives_single_call_bits(cuda, fmt):
+    """A problem's bits do not depend on what else is in its batch: the seven matrices of a layer in one
+    launch give the bits of one call each, which are within the float64 bound."""
+    made = [_packed(fmt, n, k, cuda) for n, k in LAYER]
+    run_batch, ps = made[0][2], [p for *_, p in made]
+    for m in (2, 4, 8, 16, 17, 24, 32, 33, 40, 64):
+        xs = [torch.from_numpy(synth.activations_bf16(36 + i, m, m, k).view(np.int16)).view(torch.bfloat16).to(cuda)
+              for i, (_, k) in enumerate(LAYER)]
+        ys = [torch.full((m, n), float("nan"), device=cuda) for n, _ in LAYER]
+        run_batch(xs, ps, ys)
+        for i, ((n, k), (wd, run, _, _)) in enumerate(zip(LAYER, made)):
+            # (a single GGUF call of two rows runs the M = 1 kernel)
+            assert m == 2 and fmt[0] == "q" or torch.equal(ys[i], run(xs[i], torch.float32)), (fmt, m, i)
+            x64, w64 = xs[i].double(), wd.double()
+            # as in test_split_vs_float64; the kernels of up to 32 rows round at most twice as often (f16
+            # products, a power-of-two scale per 128)
+            bound = 2 * (k / 16 + k / 32 + 10) * 2.0 ** -24 * (x64.abs() @ w64.abs().t())
+            if fmt.startswith("nf4"):
+                bound += (k / 16 * 2.0 ** -24 + 2.0 ** -17) * (x64.abs() @ w64.abs().t())
+            assert bool(((ys[i].double() - x64 @ w64.t()).abs() <= bound).all()), (fmt, m, i)
 
 
 # (m, n): one round of 96-row tiles against one or two of 128; two rounds of 128-row tiles against one
