@@ -68,21 +68,25 @@ __device__ __forceinline__ void wait_vm() {
 }
 
 // Issues this wave's 1 KB buffer->LDS loads of one slice (K bytes [k0, k0 + BK) of both panels)
-// into stage `dst`: blocks wave I .. + I of W, wave J .. + J of A (16 rows each).
+// into stage `dst`: blocks wave I .. + I of W, wave J .. + J of A (16 rows each).  The row is in the
+// vector offset (lw, la: the lane's in the wave's first block), which the range check covers whatever it
+// does with the scalar one: rows past N or M read 0.
 template <int I, int J>
 __device__ __forceinline__ void fp8_issue(__amdgpu_buffer_rsrc_t rw, __amdgpu_buffer_rsrc_t ra, uint8_t *__restrict__ dst,
-                                          int wave, int lvoff, int K, int k0) {
+                                          int wave, int lw, int la, int K, int k0) {
+    int block = kRowsPerLoad * K;
+    asm volatile("" : "+s"(block));  // the sums below stay in the loop: kept across it, they spilled the exact 256 x 256 form
 #pragma unroll
     for (int t = 0; t < I; ++t) {
         const int blk = wave * I + t;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void *)(dst + blk * 1024), 16, lvoff,
-                                                 blk * kRowsPerLoad * K + k0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void *)(dst + blk * 1024), 16,
+                                                 lw + t * block, k0, 0, 0);
     }
 #pragma unroll
     for (int t = 0; t < J; ++t) {
         const int blk = wave * J + t;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void *)(dst + Tile<I, J>::kWBytes + blk * 1024),
-                                                 16, lvoff, blk * kRowsPerLoad * K + k0, 0, 0);
+                                                 16, la + t * block, k0, 0, 0);
     }
 }
 
@@ -159,10 +163,10 @@ __device__ __forceinline__ void fp8_mma(const Fp8Frags<I, J> &f, floatx16 (&acc)
 template <bool kExact, int I, int J>
 __device__ __forceinline__ void fp8_step(const uint8_t *__restrict__ cur, uint8_t *__restrict__ nxt,
                                          bool refill, bool read_next, __amdgpu_buffer_rsrc_t rw, __amdgpu_buffer_rsrc_t ra,
-                                         int wave, int lvoff, int K, int k_next, int wn, int wm,
+                                         int wave, int lw, int la, int K, int k_next, int wn, int wm,
                                          int fr, int fc, const Fp8Frags<I, J> &f, Fp8Frags<I, J> &fn,
                                          floatx16 (&acc)[I][J]) {
-    if (refill) fp8_issue<I, J>(rw, ra, nxt, wave, lvoff, K, k_next);
+    if (refill) fp8_issue<I, J>(rw, ra, nxt, wave, lw, la, K, k_next);
     if (read_next) fp8_read_frags<I, J>(cur, wn, wm, fr, fc, fn);
     fp8_mma<kExact, I, J>(f, acc);
     if constexpr (kExact) {
@@ -228,6 +232,7 @@ void fp8_gemm_kernel(const uint8_t *__restrict__ A, const float *__restrict__ sa
     // rows, physical chunk i % kChunks, which holds logical chunk swz(row, i % kChunks).
     const int lrow = lane / kChunks;
     const int lvoff = lrow * K + swz(lrow, lane % kChunks) * 16;
+    const int lw = lvoff + wave * I * kRowsPerLoad * K, la = lvoff + wave * J * kRowsPerLoad * K;
 
     // ---- fragments: lane reads 32 bytes (2 chunks) of row lane % 32 per K=64 step ----
     const int wn = (wave / 2) * 32 * I, wm = (wave % 2) * 32 * J;
@@ -246,7 +251,7 @@ void fp8_gemm_kernel(const uint8_t *__restrict__ A, const float *__restrict__ sa
     // ring of NSTAGE slots: slot s % NSTAGE holds slice s.  All slots are filled up front.
 #pragma unroll
     for (int s = 0; s < NSTAGE; ++s)
-        if (s < KT) fp8_issue<I, J>(rw, ra, lds + s * T::kStageBytes, wave, lvoff, K, s * BK);
+        if (s < KT) fp8_issue<I, J>(rw, ra, lds + s * T::kStageBytes, wave, lw, la, K, s * BK);
 
     // slice 0's fragments: wait for this wave's slice-0 loads, then for everyone's
     Fp8Frags<I, J> fa, fb;
@@ -271,7 +276,7 @@ void fp8_gemm_kernel(const uint8_t *__restrict__ A, const float *__restrict__ sa
         const int nk = t + NSTAGE;
         // steady steps are branch-free, so the scheduler can interleave loads, reads and MFMAs
         fp8_step<kExact, I, J>(lds + ((t + 1) % NSTAGE) * T::kStageBytes, lds + (t % NSTAGE) * T::kStageBytes,
-                               kSteady || nk < KT, kSteady || t + 1 < KT, rw, ra, wave, lvoff, K, nk * BK, wn, wm, fr, fc, f,
+                               kSteady || nk < KT, kSteady || t + 1 < KT, rw, ra, wave, lw, la, K, nk * BK, wn, wm, fr, fc, f,
                                fn, acc);
     };
     int kt = 0;
@@ -414,18 +419,21 @@ constexpr int kSplitBK = 128;
 __device__ __forceinline__ int split_swz(int r, int c) { return c ^ ((r >> 1) & 7); }
 
 // This wave's loads of K bytes [k0, k0 + 128) of the tile's W and A rows into `dst` (W rows, then
-// A rows): each load brings 8 rows x 128 bytes.  Rows past the descriptors read 0.
+// A rows): each load brings 8 rows x 128 bytes.  Rows past the descriptors read 0, as does the half of
+// the last row's last chunk that K % 128 == 64 puts past them: the whole offset is in the vector offset,
+// which the range check covers whatever it does with the scalar one.  lv: the lane's offset in loads 0
+// and 1; a later pair's rows are 16 K bytes further each.
 template <int I, int J>
 __device__ __forceinline__ void split_issue(__amdgpu_buffer_rsrc_t rw, __amdgpu_buffer_rsrc_t ra, uint8_t *__restrict__ dst,
                                             const int (&lv)[2], int K, int k0) {
 #pragma unroll
     for (int t = 0; t < 4 * I; ++t)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (__attribute__((address_space(3))) void *)(dst + t * 1024), 16,
-                                                 lv[t & 1], t * 8 * K + k0, 0, 0);
+                                                 lv[t & 1] + ((t >> 1) * 16 * K + k0), 0, 0, 0);
 #pragma unroll
     for (int t = 0; t < 4 * J; ++t)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (__attribute__((address_space(3))) void *)(dst + (4 * I + t) * 1024), 16,
-                                                 lv[t & 1], t * 8 * K + k0, 0, 0);
+                                                 lv[t & 1] + ((t >> 1) * 16 * K + k0), 0, 0, 0);
 }
 
 __device__ __forceinline__ int32x8 split_frag(const uint8_t *__restrict__ rows, int r, int c) {
@@ -509,7 +517,7 @@ __global__ __launch_bounds__(64 * NW) void fp8_split_kernel(const uint8_t *__res
     // lane i of a load writes LDS bytes [16 i, 16 i + 16): row i / 8, physical chunk i % 8
     int lv[2];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) lv[u] = (lane >> 3) * K + split_swz(8 * u + (lane >> 3), lane & 7) * 16;
+    for (int u = 0; u < 2; ++u) lv[u] = (8 * u + (lane >> 3)) * K + split_swz(8 * u + (lane >> 3), lane & 7) * 16;
     const int fr = lane & 31, fc = (lane >> 5) * 2;
 
     floatx16 acc[I][J];

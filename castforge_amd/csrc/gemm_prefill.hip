@@ -595,12 +595,14 @@ void prefill_i4_kernel(PfArgs a) {
         vz[i] = row * static_cast<uint32_t>(ZW) * 4u;
     }
     // lane offsets of the x loads: load t writes rows 4 t .. 4 t + 3 of the wave's BM / NW;
-    // lane -> row 4 t + lane / 16, physical chunk lane % 16 (logical chunk ^ (row & 15))
+    // lane -> row 4 t + lane / 16, physical chunk lane % 16 (logical chunk ^ (row & 15)).  The row is in
+    // the vector offset, which the range check covers whatever it does with the scalar one: rows past M
+    // read 0.
     uint32_t lv[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const int r = kRowsX * wave + 4 * u + (lane >> 4);
-        lv[u] = static_cast<uint32_t>((lane >> 4) * K * 2 + (((lane & 15) ^ (r & 15)) * 16));
+        lv[u] = static_cast<uint32_t>(r * K * 2 + (((lane & 15) ^ (r & 15)) * 16));
     }
 
     // INT4: word t of the lane's 32 code bytes holds k = 64 h + 8 t .. + 7 of the block.
@@ -620,7 +622,7 @@ void prefill_i4_kernel(PfArgs a) {
         for (int t = 0; t < kDma; ++t)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 rx, reinterpret_cast<__attribute__((address_space(3))) void *>(reinterpret_cast<uintptr_t>(dst + t * 1024)),
-                16, lv[t & 3], (kRowsX * wave + 4 * t) * K * 2 + b * (kI4KB * 2), 0, 0);
+                16, lv[t & 3] + (t >> 2) * 32 * K, b * (kI4KB * 2), 0, 0);
     };
     auto issue_w = [&](int b, WSet &r) __attribute__((always_inline)) {
         const int g = b / bpg;

@@ -14,7 +14,8 @@
 // waves until the end, so there is no barrier in the loop:
 //   * x: each wave keeps a ring of S stages of 32 J rows x 128 bytes, filled by buffer -> LDS loads
 //     (8 rows x 128 bytes each; 16-byte pieces at piece ^ ((row >> 1) & 7), so sixteen rows read at
-//     one piece cover the 256-byte bank window; rows past M read 0);
+//     one piece cover the 256-byte bank window; rows past M read 0: the row is in the vector offset, which
+//     the range check covers whatever it does with the scalar one);
 //   * W: each lane loads its row's codes of the chunk into registers (a ring of S sets) and decodes
 //     them there: no code is decoded twice within a workgroup, because the waves' chunks differ.
 #include <algorithm>
@@ -194,13 +195,14 @@ __device__ __forceinline__ bf16x8_t decode8(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(bf16x8_t, make_uint4(pack_hi16(v[0], v[1]), pack_hi16(v[2], v[3]), pack_hi16(v[4], v[5]), pack_hi16(v[6], v[7])));
 }
 
-// XL: 1 KB loads of x per chunk (8 rows each), the size of a stage: 4 J, or fewer where M <= 8 XL
+// XL: 1 KB loads of x per chunk (8 rows each), the size of a stage: 4 J, or fewer where M <= 8 XL.
+// lv: the lane's offset in loads 0 and 1; a later pair's rows are 32 K bytes further each.
 template <int XL>
 __device__ __forceinline__ void issue_x(rsrc_t rx, uint8_t *__restrict__ dst, const int (&lv)[2], int K, int c) {
 #pragma unroll
     for (int t = 0; t < XL; ++t)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void *)(dst + t * 1024), 16, lv[t & 1],
-                                                 t * 16 * K + c * kXRow, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void *)(dst + t * 1024), 16,
+                                                 lv[t & 1] + (t >> 1) * 32 * K, c * kXRow, 0, 0);
 }
 
 // One chunk: refill stage `nxt` and set `wn` (used in the previous step) with chunk c_next, wait
@@ -358,7 +360,7 @@ __global__ __launch_bounds__(64 * NW) void qsplit_kernel(QsArgs g) {
     const rsrc_t rx = make_rsrc(a.x + static_cast<int64_t>(m0) * K, static_cast<uint32_t>(min(kBM, M - m0)) * K * 2);
     int lv[2];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) lv[u] = (lane >> 3) * K * 2 + xswz(8 * u + (lane >> 3), lane & 7) * 16;
+    for (int u = 0; u < 2; ++u) lv[u] = (8 * u + (lane >> 3)) * K * 2 + xswz(8 * u + (lane >> 3), lane & 7) * 16;
     WAddr A;
     const int row_bytes = kBytes<FMT> ? K : K / 2;
     // scales per row: GGUF planes 8 ceil(K / 32 / 8), INT4 8 ceil(G / 8)

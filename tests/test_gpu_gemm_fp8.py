@@ -185,3 +185,20 @@ def test_fp8_gemm_out_validation(cuda):
                 torch.empty((4, 8), dtype=torch.float16, device=cuda)):
         with pytest.raises(ValueError, match="out must be"):
             ops.gemm_fp8(qa, s4, qw, s8, out=bad)
+
+
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("m,n,k", [(2, 33, 192), (33, 65, 576), (520, 1050, 192), (1000, 4001, 64), (2047, 4090, 64),
+                                   (2999, 4001, 64), (4001, 4000, 64)])
+def test_fp8_operands_at_the_end_of_their_allocation(cuda, m, n, k, exact):
+    """Neither rows past M and N nor, at K % 128 == 64, bytes past the last row are read: both operands end
+    where their allocation ends, with few rows in the last tile of every tile size."""
+    def at_end(t):
+        buf = torch.empty(32 << 20, dtype=torch.uint8, device=cuda)
+        buf[-t.numel():] = t.reshape(-1)
+        return buf[-t.numel():].view(t.shape)
+
+    qa, sa = ops.quantize_fp8(torch.from_numpy(synth.fp8_inputs(87, m, m, k)).to(cuda))
+    qw, sw = ops.quantize_fp8(torch.from_numpy(synth.fp8_inputs(87, n, n, k) * np.float32(0.02)).to(cuda))
+    y = ops.gemm_fp8(at_end(qa), sa, at_end(qw), sw, out_dtype=torch.float32, exact=exact)
+    assert torch.equal(y, ops.gemm_fp8(qa, sa, qw, sw, out_dtype=torch.float32, exact=exact))

@@ -109,3 +109,32 @@ def test_prefill_tile_heights_vs_float64(cuda, fmt, m, n, monkeypatch):
     bound = (k / 16 + k / 32 + 10) * 2.0 ** -24 * mag
     y = run(x, torch.float32)
     assert bool(((y.double() - ref).abs() <= bound).all()), (fmt, m, n)
+
+
+def _at_end(t):
+    """A copy of t in the last bytes of a 32 MiB allocation of its own."""
+    b = t.contiguous().reshape(-1).view(torch.uint8)
+    buf = torch.empty(32 << 20, dtype=torch.uint8, device=t.device)
+    buf[-b.numel():] = b
+    return buf[-b.numel():].view(t.dtype).reshape(t.shape)
+
+
+@pytest.mark.parametrize("fmt", ["int4_128", "int4_32", "int8_channel", "q4_0", "q8_0", "nf4_64"])
+@pytest.mark.parametrize("prefill", [False, True])
+def test_operands_at_the_end_of_their_allocation(cuda, fmt, prefill, monkeypatch):
+    """Rows past M and N are not read: x and the codes end where their allocation ends, with tiles of every
+    kernel that hold few rows, and the results are the bits of the same operands elsewhere."""
+    if prefill:
+        monkeypatch.setenv("CASTFORGE_PREFILL_I4", "1")
+    k, n = 1152, 97
+    _, run, _, p = _packed(fmt, n, k, cuda)
+    codes = p[0] if isinstance(p, tuple) else p.codes
+    end = (_at_end(codes), p[1]) if isinstance(p, tuple) else type(p)(**{**vars(p), "codes": _at_end(codes)})
+    if isinstance(p, tuple):
+        run_end = lambda x, o: ops.gemm_w8a16(x, *end, fmt[5:], o)  # noqa: E731
+    else:
+        call = ops.gemm_w4a16 if fmt[0] == "i" else ops.gemm_nf4 if fmt[0] == "n" else ops.gemm_gguf
+        run_end = lambda x, o: call(x, end, o)  # noqa: E731
+    for m in (3, 17, 33, 65, 130, 2050):
+        x = torch.from_numpy(synth.activations_bf16(38, m, m, k).view(np.int16)).view(torch.bfloat16).to(cuda)
+        assert torch.equal(run_end(_at_end(x), torch.float32), run(x, torch.float32)), (fmt, m)
