@@ -542,12 +542,18 @@ void launch_x(QsArgs a, hipStream_t st) {
     check_launch("qsplit_kernel");
 }
 
+// Fewest rows that reach a 32-row tile of 32 I columns (qsplit_ok, launch_fmt): x stages for fewer are not built.
+template <int FMT, int I>
+constexpr int kMinRows = FMT == FMT_Q4G || FMT == FMT_Q8G ? 33 : FMT == FMT_NF4 || (FMT == FMT_I8S && I == 2) ? 17 : 2;
+
 template <int FMT, int I, int J, int NW, int S>
 void launch(const QsArgs &a, hipStream_t st) {
     if constexpr (J == 1) {
-        if (a.M <= 8) launch_x<FMT, I, J, NW, S, 1>(a, st);
-        else if (a.M <= 16) launch_x<FMT, I, J, NW, S, 2>(a, st);
-        else launch_x<FMT, I, J, NW, S, 4>(a, st);
+        if constexpr (kMinRows<FMT, I> <= 16) {
+            if (a.M <= 8) return launch_x<FMT, I, J, NW, S, 1>(a, st);
+            if (a.M <= 16) return launch_x<FMT, I, J, NW, S, 2>(a, st);
+        }
+        launch_x<FMT, I, J, NW, S, 4>(a, st);
     } else {
         launch_x<FMT, I, J, NW, S, 4 * J>(a, st);
     }
@@ -601,7 +607,8 @@ void launch_fmt(const QsArgs &a, hipStream_t st) {
     if (t32 <= (a.M <= 32 ? 3 * cus : cus) || (FMT == FMT_INT8 && a.M <= 16)) {
         launch<FMT_SMALL, 1, 1, 8, 2>(a, st);
     } else if (a.M <= 32) {
-        launch<FMT_SMALL, 2, 1, 8, 2>(a, st);
+        if constexpr (kMinRows<FMT_SMALL, 2> <= 32) launch<FMT_SMALL, 2, 1, 8, 2>(a, st);
+        else require(false, "qsplit_kernel: GGUF planes from 33 rows on");
     } else if (a.M <= 64) {
         if (tiles_of(a, 32, 64) <= cus) launch<FMT_SMALL, 1, 2, 8, 2>(a, st);
         else launch<FMT_SMALL, 2, 2, 8, 2>(a, st);
