@@ -151,9 +151,8 @@ def test_nf4_batched(cuda, block):
 @pytest.mark.parametrize("fmt", ["int4", "int8", "nf4"])
 @pytest.mark.parametrize("m", [17, 40, 64])
 def test_batched_mid_m(cuda, fmt, m):
-    """M = 17..64 in one batched launch (x tiles of 16 rows sharing each decoded weight word):
-    within tolerance of the oracle, and equal to one call per problem wherever that call runs
-    the same kernel (INT8 single calls above M = 32 run the prefill kernel)."""
+    """M = 17..64 in one batched launch of the K-split kernel: within tolerance of the oracle, and equal to
+    one call per problem."""
     shapes = [(96, 1024), (300, 2048), (64, 4096), (7, 512)]
     xs, ps, ys, refs = [], [], [], []
     for i, (n, k) in enumerate(shapes):
@@ -182,30 +181,41 @@ def test_batched_mid_m(cuda, fmt, m):
         ops.gemv_nf4_batched(xs, ps, ys)
         singles = [ops.gemm_nf4(x, p, torch.float32) for x, p in zip(xs, ps)]
     for y, y1, ref in zip(ys, singles, refs):
-        if not (fmt == "int8" and m > 32):
-            assert torch.equal(y, y1)
+        assert torch.equal(y, y1)
         _close(y, ref)
         _close(y1, ref)
 
 
-@pytest.mark.parametrize("m", [17, 40])
-@pytest.mark.parametrize("steps", [2, 3, 4, 5, 6, 9, 11])
-def test_nf4_partial_step_groups(cuda, steps, m):
-    """NF4 at M > 16 with every remainder of the K loop's groups of six 64-wide steps per K part (two
-    parts up to K = 6144), on weights no earlier call has brought into the caches: against float64."""
-    n, k = 1500, 128 * steps
-    w = torch.from_numpy(synth.weight(740 + steps, 1, n, k)).to(cuda)
-    _, x = _x(750 + steps, m, k, cuda)
-    p = ops.quantize_nf4(w, 64)
-    wd = ops.dequantize_nf4(p).cpu().double()
-    x64 = x.cpu().double()
+def _nf4_on(dev, seed, n, k):
+    """NF4 weight drawn on the device: packed, and dequantized in float64."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+    p = ops.quantize_nf4(torch.randn((n, k), generator=g, device=dev) * 0.02, 64)
+    return p, ops.dequantize_nf4(p).double()
+
+
+@pytest.mark.parametrize("m", [17, 32, 40, 64])
+@pytest.mark.parametrize("k", [256, 384, 512, 640, 768, 1152, 1408, 6208, 6400, 6464])
+def test_nf4_partial_step_groups(cuda, k, m):
+    """nf4_mfma_kernel (M = 17..64 with more than one 64 x 64 tile per CU) with every remainder of the K loop's
+    groups of six 64-wide steps per K part: 2..11 steps in two parts, 25 and 26 in four of equal and unequal
+    length (K > 6144), on weights no earlier call has brought into the caches; in a batch with a smaller
+    problem, which qsplit_kernel takes.  Both are against float64 and give the bits of their single calls."""
+    n = 64 * torch.cuda.get_device_properties(cuda).multi_processor_count + 70
+    (p, wd), (q, qd) = _nf4_on(cuda, 740 + k, n, k), _nf4_on(cuda, 741 + k, 97, k)
+    _, x = _x(750 + k, m, k, cuda)
     torch.empty(1 << 28, dtype=torch.uint8, device=cuda).zero_()  # 256 MB through the caches
-    y = ops.gemm_nf4(x, p, torch.float32).cpu().double()
-    mag = x64.abs() @ wd.abs().t()
-    # T_hi + T_lo is within 2^-17 of T, the dequantized weight within 2^-24; f32 sums: one rounding an
-    # MFMA step of 16, a scale every 64, the K parts
-    bound = (2.0 ** -17 + (k / 8 + k / 64 + 4) * 2.0 ** -24) * mag
-    assert bool(((y - x64 @ wd.t()).abs() <= bound).all())
+    y = ops.gemm_nf4(x, p, torch.float32)
+    ys = [torch.empty((m, n), device=cuda), torch.empty((m, 97), device=cuda)]
+    ops.gemv_nf4_batched([x, x], [p, q], ys)
+    assert torch.equal(ys[0], y)
+    assert torch.equal(ys[1], ops.gemm_nf4(x, q, torch.float32))
+    x64 = x.double()
+    for got, w in ((ys[0], wd), (ys[1], qd)):
+        # T_hi + T_lo is within 2^-17 of T, the dequantized weight within 2^-24; f32 sums: one rounding an
+        # MFMA step of 16, a scale every 64, the K parts or waves
+        bound = (2.0 ** -17 + (k / 8 + k / 64 + 10) * 2.0 ** -24) * (x64.abs() @ w.abs().t())
+        assert bool(((got.double() - x64 @ w.t()).abs() <= bound).all())
 
 
 def test_nf4_batched_rejects_mixed_blocks(cuda):
