@@ -21,6 +21,8 @@ and per kernel (M = 1 split-K, M = 3 and 16 skinny, M = 40 and 300 prefill):
 INT4 g128 / g64 / g32, INT8 and GGUF Q4_0 / Q8_0 run a second time with the one-MFMA prefill
 kernel forced (the *_one formats): exact (q - z) / q operands, one f32 partial per group
 (GGUF: per 32-wide block; INT8: one sum, its row scale applied once) scaled into the total.
+M = 2..64 run the K-split kernel (GGUF from 33, NF4 from 17 rows); the *_long formats have more
+groups in a row than it takes (128), and run the skinny kernel.
 """
 import os
 
@@ -130,7 +132,8 @@ def _one_mfma(call):
 
 
 FORMATS = ["int4_g128", "int4_g128_one", "int4_g64", "int4_g64_one", "int4_g32", "int4_g32_one", "int8", "int8_one",
-           "nf4", "q4_0", "q4_0_one", "q8_0", "q8_0_one"]
+           "nf4", "q4_0", "q4_0_one", "q8_0", "q8_0_one", "int4_g128_long", "int4_g64_long"]
+LONG_K = {"int4_g128_long": 16640, "int4_g64_long": 8320}  # 130 groups, 65 in each half
 MS = [1, 3, 16, 40, 300]
 
 
@@ -150,7 +153,7 @@ def _wide_x(seed, m, k):
 @pytest.mark.parametrize("m", MS)
 @pytest.mark.parametrize("fmt", FORMATS)
 def test_wide_activations_vs_oracle(cuda, fmt, m):
-    n, k = 96, 2048
+    n, k = 96, LONG_K.get(fmt, 2048)
     c = Case(fmt, n, k, cuda)
     xb = _wide_x(100 + m, m, k)
     y = c.run(_xdev(xb, cuda), torch.float32).cpu().numpy()
@@ -174,7 +177,7 @@ def test_wide_activations_vs_oracle(cuda, fmt, m):
 @pytest.mark.parametrize("m", [1, 4, 16])
 @pytest.mark.parametrize("fmt", FORMATS)
 def test_power_of_two_scale_invariance(cuda, fmt, m):
-    n, k = 80, 1024
+    n, k = 80, LONG_K.get(fmt, 1024)
     c = Case(fmt, n, k, cuda, seed=12)
     xb = _wide_x(200 + m, m, k)
     x32 = O.bf16_bits_to_f32(xb)
@@ -191,7 +194,7 @@ def test_power_of_two_scale_invariance(cuda, fmt, m):
 @pytest.mark.parametrize("m", MS)
 @pytest.mark.parametrize("fmt", FORMATS)
 def test_exact_cancellation(cuda, fmt, m):
-    n, k = 64, 2048
+    n, k = 64, LONG_K.get(fmt, 2048)
     c = Case(fmt, n, k, cuda, seed=13, halves=True)
     rng = np.random.default_rng(300 + m)
     v = rng.standard_normal((m, k // 2)).astype(np.float32)

@@ -4,7 +4,7 @@ every sampled output within |y - ref| <= 1e-3 + 1e-2 * |ref|.
 
 - NF4 block 64 at M = 64: W_gate, W_up and W_down (K = 11008) in ONE batched launch, as the
   nf4_gemm_m64 component runs it;
-- NF4 block 64 at M = 512 on W_down (4096 x 11008), the prefill kernel's 64 x 64-tile instance;
+- NF4 block 64 at M = 512 on W_down (4096 x 11008), the K-split kernel's 64 x 64 tiles;
 - W4A16 INT4 g128 at M = 16 over the whole 7-matrix block in one batched launch (config 2);
 - W4A16 INT4 g128 prefill at M = 4096 on the W_gate and W_down shapes, 64 rows x 128 columns.
 
@@ -61,7 +61,7 @@ def _int4_ref(xb, p, rows, cols):
 
 
 def test_nf4_m64_batched_mlp(cuda):
-    """nf4_gemm_m64: W_gate / W_up / W_down in one launch (skinny kernel, K up to 11008)."""
+    """nf4_gemm_m64: W_gate / W_up / W_down in one launch (the K-split kernel, K up to 11008)."""
     m = 64
     mlp = synth.LLAMA7B_BLOCK[4:]
     ps = [ops.quantize_nf4(_w(300 + i, n, k, cuda), 64) for i, (_, n, k) in enumerate(mlp)]
@@ -77,7 +77,7 @@ def test_nf4_m64_batched_mlp(cuda):
 
 
 def test_nf4_m512_w_down(cuda):
-    """nf4_gemm_m512 on W_down (4096 x 11008): the prefill kernel's 64 x 64-tile instance."""
+    """nf4_gemm_m512 on W_down (4096 x 11008): the K-split kernel's 64 x 64 tiles."""
     m, n, k = 512, 4096, 11008
     p = ops.quantize_nf4(_w(320, n, k, cuda), 64)
     xb, x = _x(321, m, k, cuda)

@@ -111,6 +111,22 @@ def test_prefill_tile_heights_vs_float64(cuda, fmt, m, n, monkeypatch):
     assert bool(((y.double() - ref).abs() <= bound).all()), (fmt, m, n)
 
 
+@pytest.mark.parametrize("m", [2, 9, 16, 24, 40, 64])
+def test_batch_over_two_kernels(cuda, m):
+    """A problem with more groups in a row than the K-split kernel takes runs on the skinny kernel, the others
+    of its batch on the K-split kernel: each gives the bits of its single call."""
+    made = [_packed("int4_128", n, k, cuda) for n, k in [(97, 1152), (70, 16640), (33, 256)]]
+    xs = [torch.from_numpy(synth.activations_bf16(39 + i, m, m, wd.shape[1]).view(np.int16)).view(torch.bfloat16).to(cuda)
+          for i, (wd, *_) in enumerate(made)]
+    ys = [torch.full((m, wd.shape[0]), float("nan"), device=cuda) for wd, *_ in made]
+    ops.gemv_w4a16_batched(xs, [p for *_, p in made], ys)
+    for x, y, (wd, run, _, _) in zip(xs, ys, made):
+        assert torch.equal(y, run(x, torch.float32))
+        x64, w64, k = x.double(), wd.double(), wd.shape[1]
+        bound = 2 * (k / 16 + k / 32 + 10) * 2.0 ** -24 * (x64.abs() @ w64.abs().t())
+        assert bool(((y.double() - x64 @ w64.t()).abs() <= bound).all()), (m, k)
+
+
 def _at_end(t):
     """A copy of t in the last bytes of a 32 MiB allocation of its own."""
     b = t.contiguous().reshape(-1).view(torch.uint8)

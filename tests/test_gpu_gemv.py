@@ -218,6 +218,36 @@ def test_nf4_partial_step_groups(cuda, k, m):
         assert bool(((got.double() - x64 @ w.t()).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("m", [2, 3, 16, 17, 33, 48, 64])
+@pytest.mark.parametrize("gran", ["channel", "tensor"])
+def test_w8a16_skinny(cuda, monkeypatch, m, gran):
+    """The INT8 skinny kernel at each of its tile counts, with row remainders: at K = 2^23, beyond the
+    K-split kernel's 32-bit offsets, and (M > 16) with that kernel turned off.  Activations of one in 2048 and
+    a power-of-two scale make every sum of the long rows an integer below 2^24: exact."""
+    for n, k in [(35, 1 << 23)] if m <= 16 else [(35, 1 << 23), (300, 1088)]:
+        monkeypatch.delenv("CASTFORGE_PREFILL_I4", raising=False)
+        if k < 1 << 23:
+            monkeypatch.setenv("CASTFORGE_PREFILL_I4", "0")
+        g = torch.Generator(device=cuda)
+        g.manual_seed(760 + m)
+        q = torch.randint(-127, 128, (n, k), generator=g, device=cuda, dtype=torch.int8)
+        s = torch.full((n if gran == "channel" else 1,), 0.5, device=cuda)
+        if k < 1 << 23:
+            _, x = _x(761, m, k, cuda)
+        else:
+            x = torch.zeros((m, k), dtype=torch.bfloat16, device=cuda)
+            x[:, 1023::2048] = torch.randint(-4, 5, (m, k // 2048), generator=g, device=cuda).to(torch.bfloat16)
+        y = torch.empty((m, n), device=cuda)
+        ops.gemv_w8a16_batched([x], [(q, s)], [y], gran)
+        cols = x.abs().amax(0) > 0
+        x64, w64 = x[:, cols].double(), q[:, cols].double() * 0.5
+        ref, mag = x64 @ w64.t(), x64.abs() @ w64.abs().t()
+        if k < 1 << 23:  # two f16 pieces of x a chunk: one rounding an MFMA step and piece, a scale every 64
+            assert bool(((y.double() - ref).abs() <= (k / 8 + k / 64 + 10) * 2.0 ** -24 * mag).all())
+        else:
+            assert float(mag.max()) < 2 ** 23 and torch.equal(y.double(), ref)
+
+
 def test_nf4_batched_rejects_mixed_blocks(cuda):
     ps = [ops.quantize_nf4(torch.zeros((16, 256), device=cuda), b) for b in (64, 32)]
     xs = [torch.zeros((1, 256), dtype=torch.bfloat16, device=cuda)] * 2

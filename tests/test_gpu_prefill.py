@@ -101,6 +101,7 @@ def test_prefill_every_tile_shape(cuda, monkeypatch, tile, fmt):
     m, n, k = 300, 328, 768
     print(f"[prefill tile] {fmt} {tile}", flush=True)
     monkeypatch.setenv("CASTFORGE_PREFILL_TILE", tile)
+    monkeypatch.setenv("CASTFORGE_NF4_MFMA", "0")  # (NF4: the variable that keeps it off its MFMA kernels)
     w = synth.weight(91, 1, n, k)
     xb, x = _x(92, m, k, cuda)
     if fmt == "int4":
