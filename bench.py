@@ -423,8 +423,8 @@ def main():
                 f"{components[f'w4a16_prefill_m{m}_n{n}_k{k}_TFLOPs']} TFLOP/s")
             del xp, yp
         nf3 = [ops.quantize_nf4(w, 64) for w in block_f32[4:]]
-        # M = 64: one launch over the three matrices on the skinny kernel, rotating over 4 copies
-        # of the weights (270 MB, beyond the 256 MB MALL); M = 512: one prefill GEMM per matrix
+        # M = 64: one launch over the three matrices on the K-split kernel, rotating over 4 copies
+        # of the weights (270 MB, beyond the 256 MB MALL); M = 512: one call per matrix
         nf3c = [nf3] + [[ops.Nf4Packed(p.codes.clone(), p.absmax.clone(), p.n, p.k, p.block) for p in nf3]
                         for _ in range(3)]
         for m in (64, 512):

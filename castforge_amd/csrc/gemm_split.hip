@@ -651,7 +651,7 @@ QsProb prob(const uint16_t *x, int64_t n, int64_t k, int64_t group, const void *
 }  // namespace
 
 // Whether qsplit_kernel takes a problem of M = m >= 2 rows.  The variables that choose a prefill
-// kernel keep M > 16 off it.
+// kernel keep M > 16 off it (NF4: CASTFORGE_NF4_MFMA=0 alone).
 bool qsplit_ok(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group, const void *codes, const void *scales) {
     if (fmt != FMT_INT4 && fmt != FMT_INT8 && fmt != FMT_NF4 && fmt != FMT_Q4G && fmt != FMT_Q8G) return false;
     // GGUF up to 32 rows: the skinny kernel, for single calls too, so that a batch gives their bits (Q8_0 / Q4_0
@@ -674,7 +674,8 @@ bool qsplit_ok(int fmt, const uint16_t *x, int64_t m, int64_t n, int64_t k, int6
     if (fmt == FMT_Q8G && group != 32) return false;
     if (fmt == FMT_INT4) {
         if (k % group != 0 || (group != 32 && group % kChunk != 0)) return false;
-        // groups of 64 and more: the largest tile's scales and zero points next to the x rings
+        // groups of 64 and more: the largest tile's scales and zero points next to the x rings, up to 128 groups
+        // (K = 8192 in groups of 64); longer rows stay on the skinny and prefill kernels
         if (group != 32 && lds_bytes<FMT_INT4, 2, 2, 8, 2, 8>(k / group) > kLdsMax) return false;
     }
     if (fmt != FMT_NF4 && m > 16 && (std::getenv("CASTFORGE_PREFILL_I4") || std::getenv("CASTFORGE_PREFILL_TILE"))) return false;

@@ -1677,7 +1677,9 @@ void launch_batch(int fmt, Problem *ps, int count, int64_t m, int y_bf16, hipStr
 // Largest M a single problem runs on the skinny kernels; beyond it the prefill kernel is
 // faster (measured on W_gate / W_up / W_down of a 7B block: INT8 and Q4_0 at M = 48 / 64 take
 // 138 / 149 and 309 / 323 us there against 103 / 100 and 200 / 197 us on the prefill kernel;
-// INT4, NF4 and Q8_0 stay faster on the skinny kernel up to M = 64).  Batched calls take the
+// INT4, NF4 and Q8_0 stay faster on the skinny kernel up to M = 64).  These are the problems that
+// qsplit_kernel has left: GGUF planes up to M = 32, NF4 up to M = 16, blocks of 32, INT4 rows of more than
+// 128 groups, K beyond its offsets, and M > 16 where a variable keeps it off.  In a batch they take the
 // skinny kernels up to M = 64 for every format.
 int64_t skinny_m_max(int fmt) { return fmt == FMT_INT8 || fmt == FMT_Q4_0 ? 32 : 64; }
 

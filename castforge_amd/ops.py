@@ -664,7 +664,8 @@ def gguf_q4_0_to_int4g(p: GgufPacked) -> Int4Packed:
 
 def gemm_gguf(x: torch.Tensor, p: GgufPacked, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """y [M, n] = x [M, k] (bf16) times decode(W)^T over GGUF planes (split-K GEMV at M = 1 and
-    2, the skinny MFMA kernel up to M = 64 (Q4_0: 32), the prefill MFMA kernel beyond)."""
+    2, the skinny MFMA kernel up to M = 32, the K-split kernel up to M = 64 and where its tiles are few,
+    the prefill MFMA kernel beyond)."""
     x = _check_x(x, p.k)
     y = torch.empty((x.shape[0], p.n), dtype=out_dtype, device=x.device)
     ffi.call("castforge_hip_gemv_gguf", p.ggml_type, _ptr(x), x.shape[0], p.n, p.k, _ptr(p.codes),

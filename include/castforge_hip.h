@@ -190,7 +190,8 @@ int32_t castforge_hip_quantize_int8_batched(const cfh_quant_problem_t *problems,
  * Replaces the evaluation of `castforge.fused_qmatmul` (passes/fuse/epilogue.rs:10-94,
  * codegen/eval.rs:1145-1179 -> eval_matmul_2d eval.rs:1465-1507, packed_rhs) and the HIP text
  * the reference emits for it (codegen/targets/gpu_c.rs:208-292, passes/loops/lower.rs:226-247).
- * M <= 64 (INT8: M <= 32) runs the MFMA decode / skinny kernels; larger M the prefill GEMM. */
+ * M = 1 runs the split-K decode kernel; from M = 2 the K-split MFMA kernel where its tiles are few (up to
+ * M = 64 always; GGUF planes from M = 33, NF4 from 17, the skinny kernel below), else the prefill GEMM. */
 int32_t castforge_hip_gemv_w4a16(const uint16_t *x, int64_t m, int64_t n, int64_t k, int64_t group,
                                  const uint32_t *codes, const uint16_t *scales_f16,
                                  const uint32_t *zeros, void *y, int32_t y_dtype, void *stream,
@@ -457,10 +458,10 @@ int32_t castforge_hip_dequantize_gguf(int32_t ggml_type, const void *codes, cons
  * dequant-GEMV of a GGUF weight: the reference decodes it to f32 (gguf.rs:513-550) and
  * evaluates the matmul (codegen/eval.rs:1465-1507).  x bf16 [m, k] 16-byte aligned; y f32 or
  * bf16.  M = 1 and 2 run the split-K MFMA kernel (one MFMA per block, scaled in f32 by its d;
- * M = 2 as two problems of one launch), M = 3..64 (Q4_0: 3..32) the skinny MFMA kernel (the
- * same per-block MFMA, x read per wave); larger M the prefill MFMA kernel
- * reading the planes directly (exact hi / lo f16 planes of the block values, which must lie
- * within f16 range); shapes neither fits take a generic kernel. */
+ * M = 2 as two problems of one launch), M = 3..32 the skinny MFMA kernel (the same per-block MFMA,
+ * x read per wave); M = 33..64, and beyond where its tiles are few, the K-split MFMA kernel and
+ * larger M the prefill MFMA kernel, both on the exact q - 8 or q with one f32 partial per block (the
+ * generic prefill form: exact bf16 terms); shapes none fits take a generic kernel. */
 int32_t castforge_hip_gemv_gguf(int32_t ggml_type, const uint16_t *x, int64_t m, int64_t n, int64_t k,
                                 const void *codes, const uint16_t *scales_f16, void *y, int32_t y_dtype,
                                 void *stream, char **out_error);
