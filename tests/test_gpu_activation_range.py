@@ -92,6 +92,13 @@ class Case:
             cd, sd = torch.from_numpy(c).to(dev), torch.from_numpy(s).to(dev)
             if fmt.endswith("_one"):  # the one-MFMA prefill kernel, forced at every M > 64
                 self.run = lambda x, out: _one_mfma(lambda: ops.gemm_w8a16(x, cd, sd, "channel", out))
+            elif fmt.endswith("_skinny"):
+                def batched(x, out):
+                    y = torch.empty((x.shape[0], n), dtype=out, device=dev)
+                    ops.gemv_w8a16_batched([x], [(cd, sd)], [y], "channel")
+                    return y
+
+                self.run = lambda x, out: _one_mfma(lambda: batched(x, out), "0")
             else:
                 self.run = lambda x, out: ops.gemm_w8a16(x, cd, sd, "channel", out)
             self.oracle = lambda xb: O.gemm_w8a16(xb, c, s)
@@ -117,11 +124,12 @@ class Case:
         self.deq = np.asarray(self.deq, np.float64).reshape(n, k)
 
 
-def _one_mfma(call):
+def _one_mfma(call, value="1"):
     """Runs call with CASTFORGE_PREFILL_I4=1: INT4 prefill problems whose groups are whole
-    128-wide K blocks take the one-MFMA kernel whatever their tile count."""
+    128-wide K blocks take the one-MFMA kernel whatever their tile count (0: none does, and M > 16
+    stays off the K-split kernel)."""
     old = os.environ.get("CASTFORGE_PREFILL_I4")
-    os.environ["CASTFORGE_PREFILL_I4"] = "1"
+    os.environ["CASTFORGE_PREFILL_I4"] = value
     try:
         return call()
     finally:
@@ -172,6 +180,13 @@ def test_wide_activations_vs_oracle(cuda, fmt, m):
         slack = ref_err + 2.0 ** -16 * (np.abs(O.bf16_bits_to_f32(xb).astype(np.float64)) @ np.abs(c.deq.T))
     far = np.abs(y - exact) > ATOL + RTOL * np.abs(exact) + slack
     assert not far.any(), f"{int(far.sum())} outputs further from the exact value than the oracle"
+
+
+@pytest.mark.parametrize("m", [20, 40, 64])
+def test_wide_activations_int8_skinny(cuda, m):
+    """The INT8 skinny kernel's two and four x tiles (batched, M > 16, the K-split kernel turned off)."""
+    test_wide_activations_vs_oracle(cuda, "int8_skinny", m)
+    test_exact_cancellation(cuda, "int8_skinny", m)
 
 
 @pytest.mark.parametrize("m", [1, 4, 16])
